@@ -268,6 +268,7 @@ __device__ __forceinline__ void epilogue_rows(const i16v (&acc)[FI][FJ], int lan
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 const int n = nw + j * 32 + 8 * q + 4 * g;
+                if (n >= N) continue;
                 const size_t at = (size_t)m * N + n;
                 if (EPI == RAW_ACC) {
                     *(i4v*)((int*)Cout + at) = (i4v){acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
@@ -346,7 +347,7 @@ __device__ __forceinline__ void epilogue_block(const i16v (&acc)[FI][FJ], const 
 #pragma unroll 4
         for (int it = 0; it < ITER; it++) {
             const int idx = t + it * NT, r = idx / CPR, c = (idx % CPR) * 8, m = m0 + r;
-            if (m < M) *(h8*)(C + (size_t)m * N + n0 + c) = *(const h8*)(tile + r * TP + c * 2);
+            if (m < M && n0 + c < N) *(h8*)(C + (size_t)m * N + n0 + c) = *(const h8*)(tile + r * TP + c * 2);
         }
         return;
     }
@@ -362,9 +363,9 @@ __device__ __forceinline__ void epilogue_block(const i16v (&acc)[FI][FJ], const 
     auto load = [&](int b, int slot) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < RB; k++) {
-            const int idx = t + (b * RB + k) * NT, r = idx / CPR, c = (idx % CPR) * 8, m = min(m0 + r, M - 1);
-            res[slot][k] = *(const h8*)(R + (size_t)m * N + n0 + c);
-            gat[slot][k] = *(const h8*)(G + (size_t)(m / L) * N + n0 + c);
+            const int idx = t + (b * RB + k) * NT, r = idx / CPR, n = min(n0 + (idx % CPR) * 8, N - 8), m = min(m0 + r, M - 1);
+            res[slot][k] = *(const h8*)(R + (size_t)m * N + n);
+            gat[slot][k] = *(const h8*)(G + (size_t)(m / L) * N + n);
         }
     };
     load(0, 0);
@@ -380,7 +381,7 @@ __device__ __forceinline__ void epilogue_block(const i16v (&acc)[FI][FJ], const 
             h8 y = *(const h8*)(tile + r * TP + c * 2);
 #pragma unroll
             for (int e = 0; e < 8; e++) y[e] = to_half((float)res[b & 1][k][e] + r16((float)gat[b & 1][k][e] * (float)y[e]));
-            if (m < M) *(h8*)(C + (size_t)m * N + n0 + c) = y;
+            if (m < M && n0 + c < N) *(h8*)(C + (size_t)m * N + n0 + c) = y;
         }
     }
 }
@@ -388,7 +389,7 @@ __device__ __forceinline__ void epilogue_block(const i16v (&acc)[FI][FJ], const 
 // int8 GEMM with direct global->LDS copies, for int8 or packed int4 weights (PER_CHANNEL, GROUP_SCALED and
 // RAW_ACC epilogues). A workgroup of NW wave64s (4 or 8) computes a BM x BN tile, the waves WGM x (NW / WGM)
 // over it (each a BM / WGM x BN / (NW / WGM) sub-tile: with four waves a BM/2 x BN/2 quarter, or with WGM = 1 all
-// BM rows and BN/4 columns) in 32x32 blocks (the products compute W A^T, so each lane ends up owning row
+// BM rows and BN/4 columns; rows past M and columns past N are computed on repeated operands and not stored) in 32x32 blocks (the products compute W A^T, so each lane ends up owning row
 // segments of C). K advances in slices of KB8
 // values through NS LDS stages: the copies of slice k + NS go out during the last k step of slice k. A stage
 // holds the slice's BM A rows (KB8 bytes each), then its BN W rows (KB8 bytes, or KB8 / 2 packed int4
@@ -408,9 +409,14 @@ __device__ __forceinline__ void epilogue_block(const i16v (&acc)[FI][FJ], const 
 //
 // One wave per SIMD (two with MINB = 2), so little else hides the issue time of copies and LDS reads: every
 // copy and fragment read is issued in the shadow of a product, spread evenly over its 32-wide k step
-// (sched_barrier pins the order). Fragments of the next k step are read during the current one; the
-// slice's barrier sits before its last k step, so the next slice's first reads start right after it.
-template <int BM, int BN, int KB8, int NS, bool W4, int EPI, int MINB, int WGM, int NW, bool IL>
+// (sched_barrier pins the order). Fragments are read RA k steps ahead; the slice's barrier sits before its last
+// RA k steps, so the next slice's first reads start right after it. RA 1 for the 256-row tiles, whose k step holds 6 or 8
+// products per wave, enough to cover an LDS read; RA 3 (a slice's fragments in registers before its products) for
+// the smaller ones, whose 1 to 6 products do not: 64 x 128, 512 x 3072 x 3072 11.1 -> 9.9 us; 128 x 128, 1101 x 3072 x 8192 33.7 ->
+// 30.4. What bounds the small tiles then is their copies, ~100 GB/s per CU (64 x 64: 0.16 us per 16 KiB slice);
+// more stages (6 to 8) measured slower, as did a k start that differs by block. The 256-row tiles are bound by power:
+// 4096 x 3072 x 3072 takes 28.7 us on zeros and 37-43 on random operands, whatever the tile.
+template <int BM, int BN, int KB8, int NS, bool W4, int EPI, int MINB, int WGM, int NW, bool IL, int RA>
 __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, const float* __restrict__ as,
                                                       const float* __restrict__ ws, const half_t* __restrict__ gs, const half_t* __restrict__ bias,
                                                       void* __restrict__ Cout, int M, int N, int K, const half_t* __restrict__ R,
@@ -423,56 +429,55 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
     constexpr int CPRB = WB / 16, RPIB = 1024 / WB, RPLB = 256 / WB;
     constexpr int STAGE = BM * KB8 + BN * WB;
     constexpr int AI = BM / (NW * RPI), BI = BN / (NW * RPIB), NI = AI + BI;  // copy instructions per wave per slice
-    static_assert((BM == 256 || BM == 128) && (WGM == 1 || WGM == 2 || WGM == 4) && NW % WGM == 0 && BN % 64 == 0 && TN % 32 == 0 && (KB8 == 64 || KB8 == 128) && BN % (NW * RPIB) == 0 &&
+    static_assert((BM == 256 || BM == 128 || BM == 64) && (WGM == 1 || WGM == 2 || WGM == 4) && NW % WGM == 0 && BN % 64 == 0 && TM % 32 == 0 && TN % 32 == 0 && (KB8 == 64 || KB8 == 128) && BN % (NW * RPIB) == 0 &&
                   BM % (NW * RPI) == 0, "tile");
     static_assert(!GRP || KB8 == 128, "one group per slice");
+    static_assert(RA >= 1 && RA <= KS && KS % (RA + 1) == 0, "a slice's k steps are a whole number of turns of the fragment ring");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int t = threadIdx.x, lane = t & 63, lq = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave / WGN, wn = wave % WGN;
 
-    // Tile order: block ids go round-robin to the 8 XCDs. When the grid allows it, XCD x gets the tiles of
-    // one (gy / 2) x (gx / 4) sub-grid, so each A row panel is read by 4 XCDs' L2s and each W panel by 2
-    // (round-robin order has every XCD read every A panel). Within the sub-grid the tiles go row by row; the
-    // eight-wave W4A8 kernel (one block per CU, 32 at a time per XCD) takes them in strips four tiles tall, column
-    // by column, so the blocks an XCD runs together cover 4 x 8 tiles rather than ~3 x 12 and read fewer panels
-    // (W4A8 4096 x 12288 x 3072: fetched bytes -13.5%, time unchanged). Sub-grids under 8 tiles wide keep rows.
-    int bx = blockIdx.x, by = blockIdx.y;
+    // Tile order: block ids go round-robin to the 8 XCDs, each with an L2 of its own. XCD x takes a contiguous eighth of the
+    // tiles in the order of strips STRIP tiles tall, column by column within a strip, so that the blocks it runs together
+    // cover a nearly square part of C and read few A and W panels through its L2. Any grid: ids that go round-robin over the
+    // columns instead have every XCD read every panel (int8, us in plain order -> strips: 2821 x 11136 x 1792 in 128 x 128 tiles
+    // 86.2 -> 62.8, 533 x 5952 x 12032 59.6 -> 43.5, in 64 x 128 96.2 -> 57.8, 641 x 704 x 10496 in 64 x 64 18.8 -> 16.6). Strips about 1024 rows tall measured best
+    // of 1 to 16 tiles; the group-scaled 128-row tiles 4 tall (4096 x 12288 x 3072: 188.1 us against 190.3 at 8).
+    constexpr int STRIP = BM == 256 || GRP ? 4 : 8;
+    int bx, by;
     {
-        const int gx = gridDim.x, gy = gridDim.y;
-        if (gx % 4 == 0 && gy % 2 == 0) {
-            const int id = by * gx + bx, x = id % 8, r = id / 8, sx = gx / 4, sy = gy / 2;
-            if (NW == 8 && GRP && sy % 4 == 0 && sx >= 8) {
-                const int strip = r / (4 * sx), w = r % (4 * sx);
-                bx = (x % 4) * sx + w / 4;
-                by = (x / 4) * sy + strip * 4 + w % 4;
-            } else {
-                bx = (x % 4) * sx + r % sx;
-                by = (x / 4) * sy + r / sx;
-            }
-        }
+        const int gx = gridDim.x, gy = gridDim.y, n = gx * gy, id = blockIdx.y * gx + blockIdx.x, x = id % 8;
+        const int strips = (gy + STRIP - 1) / STRIP, height = (gy + strips - 1) / strips;  // as even as they can be
+        const int s = x * (n / 8) + min(x, n % 8) + id / 8, strip = s / (height * gx), w = s - strip * height * gx, tall = min(height, gy - strip * height);
+        bx = w / tall;
+        by = strip * height + w - bx * tall;
     }
     const int m0 = by * BM, n0 = bx * BN;
     const int wrow = W4 ? K / 2 : K;  // bytes per W row in memory
 
     // Copy instruction j of a wave fills rows (4 j + wave) RPI .. + RPI - 1 of A (or of W, with RPIB): lane i
     // takes row (4 j + wave) RPI + i / CPR at physical chunk i % CPR, i.e. logical chunk cchunk (the swizzle
-    // term is the same for every j). A rows past M re-read row M - 1 (their results are not stored); the
-    // clamp is folded into the per-lane offsets, taken from a clamped group base so that they are never
-    // negative (they are the unsigned 32-bit voffset of the copy).
+    // term is the same for every j). A rows past M re-read row M - 1 and W rows past N row N - 1 (their results
+    // are not stored); the clamp is folded into the per-lane offsets, taken from a clamped group base so that they
+    // are never negative (they are the unsigned 32-bit voffset of the copy).
     const int crow = wave * RPI + lane / CPR, cchunk = (lane % CPR) ^ ((crow / RPL) % CPR);
     const int brow = wave * RPIB + lane / CPRB, bchunk = (lane % CPRB) ^ ((brow / RPLB) % CPRB);
-    const u32 boff = (u32)brow * wrow + bchunk * 16;
-    int arow[AI];
-    u32 aoff[AI];
+    int arow[AI], wrow0[BI];
+    u32 aoff[AI], boff[BI];
 #pragma unroll
     for (int c = 0; c < AI; c++) {
         arow[c] = min(m0 + NW * RPI * c, M - 1);
         aoff[c] = (u32)(min(m0 + NW * RPI * c + crow, M - 1) - arow[c]) * K + cchunk * 16;
     }
+#pragma unroll
+    for (int c = 0; c < BI; c++) {
+        wrow0[c] = min(n0 + NW * RPIB * c, N - 1);
+        boff[c] = (u32)(min(n0 + NW * RPIB * c + brow, N - 1) - wrow0[c]) * wrow + bchunk * 16;
+    }
     auto stage = [&](int kt) -> const char* { return smem + (kt % NS) * STAGE; };
-    // The epilogue's scales go to a scale block: ws[n0 .. n0 + BN) (BN / 64 copies of 64 floats), bias[n0 ..)
-    // (256-byte copies, lanes past BN / 2 re-read the last pair) and as[m0 .. m0 + BM) (rows past M re-read
-    // row M - 1), each copy issued by one wave. (A static LDS array of its own: the compiler can then tell the
+    // The epilogue's scales go to a scale block: ws[n0 .. n0 + BN) (BN / 64 copies of 64 floats; those past N, a
+    // multiple of 64, re-read the first), bias[n0 ..) (256-byte copies, lanes past BN / 2 or N / 2 re-read the last
+    // pair) and as[m0 .. m0 + BM) (rows past M re-read row M - 1), each copy issued by one wave. (A static LDS array of its own: the compiler can then tell the
     // epilogue's scale reads from its tile writes.)
     __shared__ __attribute__((aligned(16))) char sc[BN * 4 + SC_BIAS(BN) + BM * 4];
     if (EPI != RAW_ACC) {
@@ -481,9 +486,9 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
         for (int c = 0; c < NWS + NB + BM / 64; c++) {
             if (c % NW != wave) continue;
             if (c < NWS) {
-                dma4(ws + n0 + 64 * c, lane * 4, sc + c * 256);
+                dma4(ws + n0 + (n0 + 64 * c < N ? 64 * c : 0), lane * 4, sc + c * 256);
             } else if (c < NWS + NB) {
-                if (bias) dma4(bias + n0, (u32)min(64 * (c - NWS) + lane, BN / 2 - 1) * 4, sc + BN * 4 + (c - NWS) * 256);
+                if (bias) dma4(bias + n0, (u32)min(64 * (c - NWS) + lane, min(BN, N - n0) / 2 - 1) * 4, sc + BN * 4 + (c - NWS) * 256);
             } else {
                 const int i = c - NWS - NB, mb = min(m0 + 64 * i, M - 1);
                 dma4(as + mb, (u32)(min(m0 + 64 * i + lane, M - 1) - mb) * 4, sc + BN * 4 + SC_BIAS(BN) + i * 256);
@@ -499,7 +504,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
         // The block's scales are BN consecutive rows of gs ([N][groups], contiguous): read them in 16-byte pieces (all
         // of a thread's pieces in flight together), then transpose them into LDS.
         const half_t* src = gs + (size_t)n0 * groups;
-        const int pieces = BN * groups / 8;
+        const int pieces = min(BN, N - n0) * groups / 8;
         for (int ch = t; ch < pieces; ch += NT) {
             const h8 v = *(const h8*)(src + (size_t)ch * 8);
 #pragma unroll
@@ -512,7 +517,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
     auto copy = [&](int kt, int c) {  // copy instruction c (< NI) of slice kt
         const char* st = stage(kt);
         if (c < AI) dma16(A + (size_t)arow[c] * K + kt * KB8, aoff[c], st + (NW * c + wave) * 1024);
-        else dma16(W + (size_t)(n0 + NW * RPIB * (c - AI)) * wrow + kt * WB, boff, st + BM * KB8 + (NW * (c - AI) + wave) * 1024);
+        else dma16(W + (size_t)wrow0[c - AI] * wrow + kt * WB, boff[c - AI], st + BM * KB8 + (NW * (c - AI) + wave) * 1024);
     };
 
     // Fragment f (< FI: A block f, else W block f - FI) of k step kk: row base + lq, k values 32 kk + 16 g ..
@@ -557,7 +562,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
             for (int j = 0; j < FJ; j++) yacc[GRP ? i : 0][GRP ? j : 0] = (f16v){};
     // W4A8 with a wave over 128 rows x 32 columns (four A blocks, one W block) runs the block-major slice below.
     constexpr bool PIPE = GRP && W4 && FI == 4 && FJ == 1 && KS == 4;
-    i4v fr[2][NR];            // fragments of the current and the next k step
+    i4v fr[RA + 1][NR];       // fragments of the current k step and of the RA after it
     u2v fw[W4 ? FJ : 1];      // packed int4 W fragments of the next k step, before widening
 
     // Copy schedule: a slice's stage is free once the barrier before the slice's last k step has passed
@@ -575,10 +580,12 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
     else wait_copies();
     __syncthreads();
 #pragma unroll
-    for (int f = 0; f < NR; f++) {
-        if (PIPE) break;
-        fr[0][f] = W4 && f >= FI ? widen(wraw(stage(0), 0, f - FI)) : frag(stage(0), 0, f);
-    }
+    for (int r = 0; r < RA; r++)
+#pragma unroll
+        for (int f = 0; f < NR; f++) {
+            if (PIPE) break;
+            fr[r][f] = W4 && f >= FI ? widen(wraw(stage(0), r, f - FI)) : frag(stage(0), r, f);
+        }
     // PIPE (below): the first three products' A fragments, slice 0's packed W fragments, the first one widened. (These
     // arrays have one element in the other instantiations, which never use them; indices there are written `PIPE ? i : 0`
     // so that those instantiations compile without out-of-range constants.)
@@ -608,9 +615,10 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
         goff = (u32)(GS_OFF + (wn * TN + 4 * g) * 2);
         asm volatile("" : "+v"(goff));
     }
-    // One slice. AHEAD: slice kt + NS exists and is copied during this slice's last k step (then slices
+    // One slice. AHEAD: slice kt + NS exists and is copied during this slice's last RA k steps (then slices
     // kt + 2 .. kt + NS - 1 exist too); MORE: slice kt + 1 exists; SI >= 0: kt % NS, known at compile time,
-    // so the slice's LDS reads take their stage as an immediate offset.
+    // so the slice's LDS reads take their stage as an immediate offset; SI <= -2: not AHEAD, and -2 - SI slices after
+    // kt + 1 exist, whose copies may stay in flight.
     // GROUP_SCALED fold of block p's partial (one group: one slice) into its fp32 sums, with the group scales in gv.
     // Register r of block (i, j) is column wn TN + 32 j + 8 (r / 4) + 4 g + r % 4.
     h4v gv[GRP ? FJ : 1][4];
@@ -630,13 +638,15 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
         const char* sn = SI >= 0 ? smem + (SI + 1) % NS * STAGE : stage(kt + 1);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
-            if (ks == KS - 1) {
-                if (AHEAD) wait_copies_but<LEFT>();  // slice kt + 1 has landed
+            if (ks == KS - RA) {
+                // Slice kt + 1 has landed.
+                if constexpr (AHEAD) wait_copies_but<LEFT>();
+                else if constexpr (SI <= -2) wait_copies_but<(-2 - SI) * NI>();
                 else wait_copies();
                 __syncthreads();
             }
-            const int cur = ks & 1, nxt = cur ^ 1;
-            const bool last = ks == KS - 1;
+            const int cur = ks % (RA + 1), nxt = (ks + RA) % (RA + 1);
+            const bool last = ks >= KS - RA;  // the fragments read now are the next slice's
 #pragma unroll
             for (int p = 0; p < NF; p++) {
                 // GROUP_SCALED: the previous slice's partial of block p is folded just before the block's first
@@ -645,10 +655,10 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
                 if (GRP && ks == 0 && kt > 0) fold(p);
                 const i16v c0 = GRP && ks == 0 ? (i16v){} : acc[p / FJ][p % FJ];
                 acc[p / FJ][p % FJ] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[cur][FI + p % FJ], fr[cur][p / FJ], c0, 0, 0, 0);
-                if (AHEAD && ks == KS - 1)
+                if (AHEAD && last)
 #pragma unroll
                     for (int c = 0; c < NI; c++)
-                        if (c * NF / NI == p) copy(kt + NS, c);
+                        if (c * NF * RA / NI == (ks - (KS - RA)) * NF + p) copy(kt + NS, c);
                 if (GRP && ks == 0 && p == NF - 1)  // this slice's scales, once the previous slice's are used
 #pragma unroll
                     for (int j = 0; j < FJ; j++)
@@ -657,9 +667,11 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
                 if (!last || MORE) {
 #pragma unroll
                     for (int f = 0; f < NR; f++) {
-                        if ((RD(f) * NF + NF / 2) / NR != p) continue;
-                        if (W4 && f >= FI) fw[W4 ? f - FI : 0] = last ? wraw(sn, 0, f - FI) : wraw(st, ks + 1, f - FI);
-                        else fr[nxt][f] = last ? frag(sn, 0, f) : frag(st, ks + 1, f);
+                        // One k step ahead: spread over the step's products; further ahead: at its start, since the wave
+                        // holds few products to spread them over.
+                        if ((RD(f) * NF + (RA == 1 ? NF / 2 : 0)) / NR != p) continue;
+                        if (W4 && f >= FI) fw[W4 ? f - FI : 0] = last ? wraw(sn, ks + RA - KS, f - FI) : wraw(st, ks + RA, f - FI);
+                        else fr[nxt][f] = last ? frag(sn, ks + RA - KS, f) : frag(st, ks + RA, f);
                     }
                     if (W4 && p == NF - 1)
 #pragma unroll
@@ -749,7 +761,20 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
         }
     }
     for (; kt + NS < KT; kt++) run(kt, yes{}, yes{}, any{});
-    for (; kt + 1 < KT; kt++) run(kt, no{}, yes{}, any{});
+    if constexpr (RA > 1 && !PIPE) {
+        // The last slices: each waits for its successor only (a wait for all copies would drain the NS - 2 slices behind it).
+        auto tail = [&](auto self, auto left) __attribute__((always_inline)) {
+            constexpr int LEFT_S = decltype(left)::value;  // slices after kt + 1
+            if (kt + 1 + LEFT_S < KT) {
+                run(kt, no{}, yes{}, std::integral_constant<int, -2 - LEFT_S>{});
+                kt++;
+            }
+            if constexpr (LEFT_S > 0) self(self, std::integral_constant<int, LEFT_S - 1>{});
+        };
+        tail(tail, std::integral_constant<int, NS - 2>{});
+    } else {
+        for (; kt + 1 < KT; kt++) run(kt, no{}, yes{}, any{});
+    }
     run(kt, no{}, no{}, any{});
     if constexpr (PIPE) {  // the last slice's blocks 2 and 3
 #pragma unroll
@@ -782,7 +807,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
     }
 }
 
-template <int BM, int BN, int KB8, int NS, bool W4, int EPI, int MINB = 1, int WGM = 2, int NW = 4, bool IL = false>
+template <int BM, int BN, int KB8, int NS, bool W4, int EPI, int MINB = 1, int WGM = 2, int NW = 4, bool IL = false, int RA = 1>
 static int launch_gemm8(const void* a, const void* w, const float* as, const float* ws, const void* gs, const void* bias, void* c, int M, int N, int K,
                         const void* R, const void* G, int L, void* stream) {
     const size_t stage = (size_t)BM * KB8 + (size_t)BN * (W4 ? KB8 / 2 : KB8);
@@ -790,17 +815,77 @@ static int launch_gemm8(const void* a, const void* w, const float* as, const flo
     size_t lds = EPI == RAW_ACC || stages > tile ? stages : tile;  // dynamic part; the scale block is static
     if (EPI == GROUP_SCALED) lds = (lds + 15) / 16 * 16 + (size_t)BN * (K / KB8) * 2;
     if (lds > 160 * 1024 / MINB - (size_t)(BN * 4 + SC_BIAS(BN) + BM * 4)) return -1;
-    auto kern = gemm8_kernel<BM, BN, KB8, NS, W4, EPI, MINB, WGM, NW, IL>;
+    auto kern = gemm8_kernel<BM, BN, KB8, NS, W4, EPI, MINB, WGM, NW, IL, RA>;
     static std::atomic<size_t> configured[RDA_MAX_DEVICES];
     if (const int e = ensure_dynamic_lds((const void*)kern, lds, configured)) return e;
-    hipLaunchKernelGGL(kern, dim3(N / BN, (M + BM - 1) / BM), dim3(64 * NW), lds, (hipStream_t)stream, (const int8_t*)a, (const int8_t*)w, as, ws,
+    hipLaunchKernelGGL(kern, dim3((N + BN - 1) / BN, (M + BM - 1) / BM), dim3(64 * NW), lds, (hipStream_t)stream, (const int8_t*)a, (const int8_t*)w, as, ws,
                        (const half_t*)gs, (const half_t*)bias, c, M, N, K, (const half_t*)R, (const half_t*)G, L);
     return (int)hipGetLastError();
 }
 
-// Tile width for the direct-copy kernel: the one of 256, 192, 128 that divides N and leaves the fewest idle
-// CU slots in the last round of 256-CU waves (ties to the wider tile); 0 if none divides N.
-static int gemm8_width(int M, int N) {
+// A tile the direct-copy kernel is built with for 128-value slices, and what a launch of it costs: `fixed` us outside
+// the K loop, and per 128-value slice s0 us with up to half of the CUs busy, s1 with every CU holding one workgroup (the
+// L2s and the power budget are shared; linear in between) and, where two fit a CU, s2 with two each.
+struct TileCost {
+    int bm, bn, resident;
+    float fixed, s0, s1, s2;
+};
+
+// Least-squares fits to the measured times of 133 int8, 71 int4 and 74 group-scaled shapes (M 64-8192, N 512-12288, K
+// 1024-12288, and the DiT's own), every tile on every shape; the rule below then picks a tile within 0.8%, 2.0% and 1.1%
+// (geometric means) of the fastest one for the shape. No one tile does: 512 x 3072 x 3072 (int8) takes 9.9 us in
+// 64 x 128 tiles, 13.0 in 128 x 128, 26 in 256 x 192 and 32 in 256 x 256 (24 to 32 workgroups for 256 CUs); 1101 x 3072 x 8192
+// 30.1 us in 128 x 128 and 59 in 256 x 192; 4096 x 3072 x 3072 38.5 us in 256 x 192 and 61 in 64 x 64.
+constexpr TileCost I8_TILES[] = {
+    {256, 256, 1, 6.66f, 1.05f, 1.77f, 0.f}, {256, 192, 1, 6.04f, 0.84f, 1.33f, 0.f},   {128, 192, 1, 6.00f, 0.45f, 0.70f, 0.f},
+    {128, 128, 1, 4.67f, 0.33f, 0.49f, 0.f}, {128, 128, 2, 3.12f, 0.56f, 0.71f, 0.93f}, {64, 128, 1, 2.73f, 0.26f, 0.31f, 0.f},
+    {64, 64, 2, 2.52f, 0.18f, 0.21f, 0.36f},
+};
+constexpr TileCost I4_TILES[] = {
+    {128, 256, 1, 6.03f, 0.52f, 0.73f, 0.f}, {128, 128, 2, 5.14f, 0.31f, 0.42f, 0.73f}, {64, 128, 2, 4.16f, 0.23f, 0.27f, 0.46f}, {64, 64, 2, 3.05f, 0.21f, 0.25f, 0.28f},
+};
+// The last one only where no other's staged group scales fit in LDS (K past ~31000).
+constexpr TileCost GROUP_TILES[] = {
+    {128, 128, 2, 5.25f, 0.54f, 0.70f, 1.18f}, {128, 256, 1, 5.90f, 0.86f, 1.17f, 0.f}, {64, 128, 2, 3.83f, 0.35f, 0.39f, 0.66f},
+    {64, 64, 2, 2.92f, 0.31f, 0.33f, 0.41f},   {128, 128, 1, 1e6f, 0.54f, 0.73f, 0.f},
+};
+
+// Estimated us of an (M, N, K) product in tiles of t on 256 CUs: whole rounds of the workgroups the chip holds, then the
+// remainder's round at its occupancy. With two per CU, one CU with two already makes the round nearly as long as all.
+static float tile_us(const TileCost& t, int M, int N, int K) {
+    constexpr int CUS = 256;
+    const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), round = (long)CUS * t.resident;
+    const float slices = (float)(K / 128);
+    auto slice = [&](long n) {
+        const float busy = (float)n / CUS;
+        if (n > CUS) return t.s2 * (0.7f + 0.15f * busy);
+        return t.s0 + (t.s1 - t.s0) * (busy > 0.5f ? 2.f * busy - 1.f : 0.f);
+    };
+    float us = (float)(tiles / round) * (t.fixed + slices * slice(round));
+    if (tiles % round) us += t.fixed + slices * slice(tiles % round);
+    return us;
+}
+
+// The tile of `tiles` with the least estimated time among those not in `tried` (a bit per tile); marks it. -1 if none is left.
+template <int COUNT>
+static int best_tile(const TileCost (&tiles)[COUNT], unsigned& tried, int M, int N, int K) {
+    int best = -1;
+    float least = 0.f;
+    for (int i = 0; i < COUNT; i++) {
+        if (tried >> i & 1) continue;
+        const float us = tile_us(tiles[i], M, N, K);
+        if (best < 0 || us < least) {
+            best = i;
+            least = us;
+        }
+    }
+    if (best >= 0) tried |= 1u << best;
+    return best;
+}
+
+// Tile width for int8 weights in 64-value slices (K % 128 == 64): the one of 256, 192, 128 that divides N and leaves the
+// fewest idle CU slots in the last round of 256-CU waves (ties to the wider tile); 0 if none divides N.
+static int narrow_slice_width(int M, int N) {
     int best = 0;
     double best_util = 0.0;
     for (int bn : {256, 192, 128}) {
@@ -825,44 +910,56 @@ static int dispatch8(const void* a, const void* w, const float* as, const float*
     auto aligned = [](const void* p, uintptr_t al) { return ((uintptr_t)p & (al - 1)) == 0; };
     // A and W reach LDS by 16-byte global->LDS copies (rows stay aligned: K % 64 == 0).
     if (!aligned(a, 16) || !aligned(w, 16) || !aligned(c, 16) || !aligned(ws, 16) || !aligned(bias, 8) || !aligned(R, 8) || !aligned(G, 8)) return -1;
+#define RDA_TILE(...) launch_gemm8<__VA_ARGS__>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream)
+    unsigned tried = 0;
     if constexpr (EPI == GROUP_SCALED) {
-        // One group per 128-wide slice. 128 x 128 blocks of four waves leave room for two blocks per CU, so one
-        // block's group folds (vector ALU) overlap the other's products. Each wave takes all 128 rows and 32 columns:
-        // one int4 fragment to widen per k step instead of two (as 64 x 64), for two more A fragment reads from LDS.
-        // The block's group scales are staged whole (BN x K / 128 halves), so past K = 3456 two blocks no longer fit
-        // a CU's LDS: there, with N % 256 == 0, one 128 x 256 block of eight waves per CU (each A panel serving 256
-        // columns), else one 128 x 128 block, which holds the scales of K up to ~45000. In one process:
-        // 4096 x 12288 x 3072 197.0 / 198.6 us two 128 x 128 blocks per CU, 200.9 / 202.3 one 128 x 256, 217.6 one
-        // 128 x 128; 4096 x 3072 x 12288 210.8 one 128 x 256 (four stages 213.4 at two; one 128 x 128 234-239).
-        if (group != 128 || K % 128 != 0 || N % 128 != 0 || !aligned(gs, 16)) return -1;
-        {
-            const int e = launch_gemm8<128, 128, 128, 3, W4, EPI, 2, 1, 4, IL>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream);
+        // One group per 128-wide slice. The tiles of 128 rows give each wave all of them and 32 columns (one int4
+        // fragment to widen per k step) in the block-major slice, whose folds run beside the products; two 128 x 128
+        // blocks fit a CU up to K = 3456 (the block's group scales are staged whole: BN x K / 128 halves), past that one
+        // 128 x 256 block of eight waves. Fewer rows: tiles of 64, fragments read a slice ahead. 4096 x 12288 x 3072: 200.2 us
+        // in 128 x 256, 201.0 in 128 x 128, 231.7 in 64 x 128; 512 x 3072 x 12288: 38.0 in 64 x 128, 41.5 in 64 x 64, 60 before.
+        if (group != 128 || K % 128 != 0 || !aligned(gs, 16)) return -1;
+        if (IL && N % 128 != 0) return -1;
+        for (int i; (i = best_tile(GROUP_TILES, tried, M, N, K)) >= 0;) {
+            int e = -1;
+            switch (i) {
+            case 0: e = RDA_TILE(128, 128, 128, 3, W4, EPI, 2, 1, 4, IL); break;
+            case 1: e = RDA_TILE(128, 256, 128, 3, W4, EPI, 1, 1, 8, IL); break;
+            case 2: e = RDA_TILE(64, 128, 128, 3, W4, EPI, 2, 1, 4, IL, 3); break;
+            case 3: e = RDA_TILE(64, 64, 128, 4, W4, EPI, 2, 2, 4, IL, 3); break;
+            case 4: e = RDA_TILE(128, 128, 128, 3, W4, EPI, 1, 1, 4, IL); break;
+            }
             if (e >= 0) return e;
         }
-        if (N % 256 == 0) {
-            const int e = launch_gemm8<128, 256, 128, 3, W4, EPI, 1, 1, 8, IL>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream);
-            if (e >= 0) return e;
+        return -1;
+    } else if constexpr (W4) {
+        if (K % 128 != 0) return -1;
+        switch (best_tile(I4_TILES, tried, M, N, K)) {
+        case 0: return RDA_TILE(128, 256, 128, 3, true, EPI, 1, 1, 8, false, 3);
+        case 1: return RDA_TILE(128, 128, 128, 3, true, EPI, 2, 1, 4, false, 3);
+        case 2: return RDA_TILE(64, 128, 128, 4, true, EPI, 2, 1, 4, false, 3);
+        default: return RDA_TILE(64, 64, 128, 4, true, EPI, 2, 2, 4, false, 3);
         }
-        return launch_gemm8<128, 128, 128, 3, W4, EPI, 1, 1, 4, IL>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream);
     } else {
-        // 128-value k slices when K allows (two stages, three for 128-wide tiles), else 64 in four stages.
-        const bool wide = K % 128 == 0;
-        if (W4 && !wide) return -1;
-        switch (gemm8_width(M, N) * 2 + (wide ? 1 : 0)) {
-            // int8 weights: eight waves of 64 x 128 (4096 x 8192 x 3072: 91.1-92.3 -> 88.4-90.0 us on one box).
-            case 513:
-                if constexpr (!W4) return launch_gemm8<256, 256, 128, 2, false, EPI, 1, 4, 8>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream);
-                else return launch_gemm8<256, 256, 128, 2, W4, EPI>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream);
-            // int8 weights: eight waves of 64 x 96 (two per SIMD, so one wave's fragment and copy waits are covered by the
-            // other's products: 39.7 -> 38.6 us at 4096 x 3072 x 3072); int4 weights keep four waves of 128 x 96.
-            case 385: return launch_gemm8<256, 192, 128, 2, W4, EPI, 1, (W4 ? 2 : 4), (W4 ? 4 : 8)>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream);
-            case 257: return launch_gemm8<256, 128, 128, 3, W4, EPI>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream);
-            case 512: if constexpr (!W4) return launch_gemm8<256, 256, 64, 4, false, EPI>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream); return -1;
-            case 384: if constexpr (!W4) return launch_gemm8<256, 192, 64, 4, false, EPI>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream); return -1;
-            case 256: if constexpr (!W4) return launch_gemm8<256, 128, 64, 4, false, EPI>(a, w, as, ws, gs, bias, c, M, N, K, R, G, L, stream); return -1;
-            default: return -1;
+        if (K % 128 == 0) {
+            switch (best_tile(I8_TILES, tried, M, N, K)) {
+            case 0: return RDA_TILE(256, 256, 128, 2, false, EPI, 1, 4, 8);
+            case 1: return RDA_TILE(256, 192, 128, 2, false, EPI, 1, 4, 8);
+            case 2: return RDA_TILE(128, 192, 128, 3, false, EPI, 1, 2, 4, false, 3);
+            case 3: return RDA_TILE(128, 128, 128, 4, false, EPI, 1, 2, 4, false, 3);
+            case 4: return RDA_TILE(128, 128, 128, 2, false, EPI, 2, 2, 4, false, 3);
+            case 5: return RDA_TILE(64, 128, 128, 4, false, EPI, 1, 2, 8, false, 3);
+            default: return RDA_TILE(64, 64, 128, 4, false, EPI, 2, 2, 4, false, 3);
+            }
+        }
+        switch (narrow_slice_width(M, N)) {
+        case 256: return RDA_TILE(256, 256, 64, 4, false, EPI, 1, 4, 8);
+        case 192: return RDA_TILE(256, 192, 64, 4, false, EPI);
+        case 128: return RDA_TILE(256, 128, 64, 4, false, EPI);
+        default: return -1;
         }
     }
+#undef RDA_TILE
 }
 
 template <int BM, int BN, int WM, int WN, bool W4, int EPI>

@@ -205,22 +205,62 @@ def test_blockmajor_model_catches_mistakes(NS):
     assert run_schedule_blockmajor(NS, KT, copy_from=12)
 
 
+def run_schedule_ahead(NS, KT, NI=4, RA=3, KS=4, barrier_at=None, copy_from=None, tail_left=0):
+    """Fragments read RA k steps ahead (the small tiles): the prologue reads slice 0's first RA steps, k step ks the
+    fragments of step ks + RA (the next slice's from step KS - RA on); the wait and barrier sit before step KS - RA, the copies
+    of slice kt + NS go out over the last RA steps. Past the last copies a slice waits for its successor only: the slices
+    after that (tail_left more, for a planted mistake) may still be in flight."""
+    m = Model(NS, KT, NI)
+    barrier_at = KS - RA if barrier_at is None else barrier_at
+    copy_from = KS - RA if copy_from is None else copy_from
+    for s in range(min(NS, KT)):
+        m.copy(s, NI)
+    m.wait((NS - 1) * NI if KT >= NS else 0)
+    m.barrier()
+    m.read(0)
+    for kt in range(KT):
+        ahead, more = kt + NS < KT, kt + 1 < KT
+        for ks in range(KS):
+            if ks == barrier_at:
+                m.wait((NS - 2) * NI if ahead else max(0, KT - 2 - kt + tail_left) * NI)
+                m.barrier()
+            if ahead and ks == copy_from:
+                m.copy(kt + NS, NI)
+            if ks + RA < KS:
+                m.read(kt)
+            elif more:
+                m.read(kt + 1)
+    if set(m.last_read) != set(range(KT)):
+        m.errors.append("not every slice was read")
+    return m.errors
+
+
+@pytest.mark.parametrize("NS", [2, 3, 4])
+@pytest.mark.parametrize("KT", list(range(1, 13)) + [24, 64])
+def test_ahead_schedule_is_race_free(NS, KT):
+    assert run_schedule_ahead(NS, KT) == []
+
+
+@pytest.mark.parametrize("NS", [2, 3, 4])
+def test_ahead_model_catches_mistakes(NS):
+    assert run_schedule_ahead(NS, 10, barrier_at=2)  # the next slice's first read before its copies are known to have landed
+    assert run_schedule_ahead(NS, 10, copy_from=0)  # copies before the barrier: this slice's last read may be outstanding
+    assert run_schedule_ahead(NS, 10, tail_left=1)  # a tail wait one slice too loose
+
+
 def tile_of(block, gx, gy, strips):
-    """gemm8_kernel's block remap: block id -> (bx, by). Ids go round-robin to the 8 XCDs; XCD x takes the
-    (gy / 2) x (gx / 4) sub-grid x, row by row, or (strips: the eight-wave W4A8 kernel, sub-grids at least 8 tiles wide)
-    in strips four tiles tall, column by column."""
-    by, bx = divmod(block, gx)
-    if gx % 4 or gy % 2:
-        return bx, by
-    x, r, sx, sy = block % 8, block // 8, gx // 4, gy // 2
-    if strips and sy % 4 == 0 and sx >= 8:
-        strip, w = divmod(r, 4 * sx)
-        return (x % 4) * sx + w // 4, (x // 4) * sy + strip * 4 + w % 4
-    return (x % 4) * sx + r % sx, (x // 4) * sy + r // sx
+    """gemm8_kernel's block remap: block id -> (bx, by). Ids go round-robin to the 8 XCDs; XCD x takes a contiguous eighth
+    of the tiles in strips at most 4 tiles tall (strips: the 256-row and the W4A8 tiles) or 8, as even as they can be,
+    column by column."""
+    n, x, most = gx * gy, block % 8, 4 if strips else 8
+    tall = -(-gy // -(-gy // most))
+    strip, w = divmod(x * (n // 8) + min(x, n % 8) + block // 8, tall * gx)
+    h = min(tall, gy - strip * tall)
+    return w // h, strip * tall + w % h
 
 
 @pytest.mark.parametrize("strips", [False, True])
-@pytest.mark.parametrize("gx,gy", [(48, 32), (12, 16), (16, 16), (4, 8), (8, 4), (96, 32), (6, 3), (5, 8)])
+@pytest.mark.parametrize("gx,gy", [(48, 32), (24, 9), (1, 1), (3, 17), (87, 23), (12, 16), (16, 16), (4, 8), (8, 4), (96, 32), (6, 3), (5, 8)])
 def test_tile_order_is_a_permutation(gx, gy, strips):
     tiles = [tile_of(b, gx, gy, strips) for b in range(gx * gy)]
     assert sorted(tiles) == sorted((x, y) for x in range(gx) for y in range(gy))

@@ -253,7 +253,7 @@ def test_w8a8_linear_bit_exact(dev, M, N, K, group, bias):
     assert_same(bits(out), bits(ref))
 
 
-# 128-, 192- and 256-wide tiles of the direct-copy GEMM; N = 320 (no such width divides it) takes the register-load GEMM
+# whole and partial column tiles of the direct-copy GEMM
 @pytest.mark.parametrize("B,L,K,N", [(2, 300, 512, 256), (1, 600, 256, 576), (2, 2048, 256, 8192), (1, 520, 256, 320)])
 def test_gemm_residual_epilogue_bit_exact(dev, B, L, K, N):
     print(f"residual epilogue B={B} L={L} K={K} N={N}", flush=True)
@@ -383,6 +383,53 @@ def test_w4a8_interleaved_gemm_refuses_other_shapes(dev):
     assert not int8_gemm._interleaved(w, torch.ones(N, K // 128, dtype=torch.float16, device=dev), None, N, K, True, 128)
 
 
+# One shape per tile of the direct-copy GEMM's rule, each with a partial last row tile and (past 64-wide tiles) a partial
+# last column tile; K / 128 = 1, 2, 3, 5, 7 and 12 slices: fewer than the stages, as many, whole passes and tails.
+@pytest.mark.parametrize("M,N,K", [(5, 64, 384), (323, 2880, 640), (659, 3008, 896), (659, 3008, 128), (1286, 3008, 1536), (3352, 2368, 128),
+                                   (3862, 3136, 256)])
+def test_int8_tiles_bit_exact(dev, M, N, K):
+    """64 x 64, 64 x 128, 128 x 128 (one and two per CU), 128 x 192, 256 x 192 and 256 x 256 tiles, in this order, with a
+    bias and with the gated residual."""
+    print(f"int8 tiles M={M} N={N} K={K}", flush=True)
+    x, w, ws = activations(M, K, seed=81), int8_weights(N, K, seed=82), channel_scales(N, seed=83)
+    b = (torch.randn(N, generator=gen(84)) * 0.5).half()
+    q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), group=128)
+    acc = oracle.gemm_acc(q_ref, w.numpy())
+    xd, wd, wsd = x.to(dev), w.to(dev), ws.to(dev)
+    out = int8_gemm.linear(xd, wd, wsd, b.to(dev), rotate=True, group=128)
+    assert_same(bits(out), bits(oracle.gemm_epilogue(acc, s_ref, ws.numpy(), b.numpy())))
+    B = 2 if M % 2 == 0 else 1
+    R, G = torch.randn(B, M // B, N, generator=gen(85)).half(), torch.randn(B, N, generator=gen(86)).half()
+    out = int8_gemm.linear(xd, wd, wsd, None, rotate=True, res=(R.to(dev), G.to(dev)), group=128)
+    assert_same(bits(out), bits(oracle.gemm_epilogue(acc, s_ref, ws.numpy(), R=R.numpy().reshape(M, N), G=G.numpy(), L=M // B)))
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 576, 256), (672, 3008, 256), (2692, 1472, 256), (4159, 960, 1280)])
+def test_int4_tiles_bit_exact(dev, M, N, K):
+    """W4A4 in 64 x 64, 64 x 128, 128 x 128 and 128 x 256 tiles, in this order, partial last tiles both ways."""
+    print(f"int4 tiles M={M} N={N} K={K}", flush=True)
+    x, ws = activations(M, K, seed=91), channel_scales(N, seed=93)
+    w, wp = int4_weights(N, K, seed=92)
+    k = kern()
+    out = int8_gemm.run(k.rot_quant_pack_a_i4, k.gemm_i4, x.to(dev), wp.to(dev), ws.to(dev), None, K)
+    q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), i4=True)
+    assert_same(bits(out), bits(oracle.gemm_epilogue(oracle.gemm_acc(q_ref, w.numpy()), s_ref, ws.numpy())))
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 64, 384), (659, 3008, 128), (4110, 960, 128), (1863, 2240, 640), (1666, 1280, 640), (70, 256, 12288)])
+def test_group_scaled_tiles_bit_exact(dev, M, N, K):
+    """W4A8 in 64 x 64, 64 x 128, 128 x 128 and 128 x 256 tiles with partial last tiles, in natural order (N % 128 == 64),
+    then k-interleaved 64 x 128 and 64 x 64 tiles."""
+    print(f"group-scaled tiles M={M} N={N} K={K}", flush=True)
+    x = activations(M, K, seed=95, outliers=0)
+    w, wp = int4_weights(N, K, seed=96)
+    gs = (torch.rand(N, K // 128, generator=gen(97)) * 1.5e-2 + 5e-3).half()
+    b = (torch.randn(N, generator=gen(98)) * 0.5).half()
+    out = int8_gemm.linear_w4a8(x.to(dev), wp.to(dev), gs.to(dev), b.to(dev), group=128)
+    q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), group=128)
+    assert_same(bits(out), bits(oracle.w4a8_epilogue(oracle.w4a8_partials(q_ref, w.numpy()), s_ref, gs.numpy(), b.numpy())))
+
+
 def test_w4a4_hook_path_bit_exact(dev):
     """rot_quant_pack_a_i4 + gemm_i4 (the convrot_w4a4_forward replacement) against the oracle."""
     M, N, K = 600, 256, 1024
@@ -482,8 +529,7 @@ def test_linears_take_strided_activations(dev, layout):
 @pytest.mark.parametrize("seed", range(10))
 def test_linears_random_shapes(dev, seed):
     """Seeded random shapes through both linears, each against the oracle bit for bit: M from 1 to 1200 rows (partial
-    row tiles, and fewer rows than one tile), N a multiple of 64 up to 1280 (tile widths of 64 to 256, or none of them,
-    which takes the register-load GEMM), K a multiple of the rotation group up to 4096, bias on half the cases."""
+    row tiles, and fewer rows than one tile), N a multiple of 64 up to 1280 (whole and partial column tiles), K a multiple of the rotation group up to 4096, bias on half the cases."""
     rng = np.random.default_rng(2000 + seed)
     M = int(rng.integers(1, 1201))
     N = 64 * int(rng.integers(1, 21))
