@@ -98,8 +98,14 @@ def load():
     return _lib
 
 
+def raw_stream():
+    """torch's current stream on the current device, as an integer: what the entry points launch on. (torch.cuda.current_stream()
+    builds a Stream object behind several device lookups: 3.0 us a call against 0.2.)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(raw_stream())
 
 
 def ptr(t):
@@ -108,7 +114,7 @@ def ptr(t):
 
 def call(name, *args):
     """Calls an entry point with the current stream appended and checks its status."""
-    check(getattr(load(), name)(*args, stream()))
+    check(getattr(load(), name)(*args, raw_stream()))
 
 
 def long_array(values):

@@ -37,7 +37,7 @@ class Kernels:
 def launch(func, grid_x, grid_y, block, args, shared=0):
     """Calls entry point ``func`` with ``args`` on the current stream. The grid, block and LDS size
     of the reference's call are accepted for compatibility; the library sizes its own launch."""
-    check(func(*args, _lib.stream()))
+    check(func(*args, _lib.raw_stream()))
 
 
 kernels = None
@@ -65,13 +65,13 @@ def attention(q, k, v, out, scale, int8_qk=False):
         return
     k, v = (t if _dma_ready(t) else t.clone(memory_format=torch.contiguous_format) for t in (k, v))
     strides = _lib.long_array([*q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3]])
-    p = _lib.ptr
+    stream = _lib.raw_stream()
     if int8_qk:
         workspace = torch.empty(kernels.attn_i8_workspace(b, kv_heads, k_len), dtype=torch.uint8, device=q.device)
-        launch(kernels.pack_k_i8, 0, 0, 0, [p(k), p(workspace), b, kv_heads, k_len, *k.stride()[:3]])
-        launch(kernels.attn_i8, 0, 0, 0, [p(q), p(workspace), p(v), p(out), b, heads, kv_heads, q_len, k_len, strides, scale])
+        check(kernels.pack_k_i8(k.data_ptr(), workspace.data_ptr(), b, kv_heads, k_len, *k.stride()[:3], stream))
+        check(kernels.attn_i8(q.data_ptr(), workspace.data_ptr(), v.data_ptr(), out.data_ptr(), b, heads, kv_heads, q_len, k_len, strides, scale, stream))
     else:
-        launch(kernels.attn, 0, 0, 0, [p(q), p(k), p(v), p(out), b, heads, kv_heads, q_len, k_len, strides, scale])
+        check(kernels.attn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, heads, kv_heads, q_len, k_len, strides, scale, stream))
 
 
 def scale_log2(scale):

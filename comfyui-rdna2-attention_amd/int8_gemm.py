@@ -79,21 +79,35 @@ def _dense(x):
 def quantize(quant, x, K, up=None, group=ROT_GROUP):
     """Runs one activation -> rotate -> quantize entry point. x is (M, K) fp16, or (M, 2K) for situ; any strides
     (layouts the kernels cannot address are copied first). Returns (packed, scales)."""
-    k = get_kernels()
+    get_kernels()
+    packed_a, a_scale = quantized(x.shape[0], K, x.device)
+    _quantize_to(quant, x, K, up, group, packed_a.data_ptr(), a_scale.data_ptr(), _lib.raw_stream())
+    return packed_a, a_scale
+
+
+def _quantize_to(quant, x, K, up, group, codes, scales, stream):
+    """quantize() into device addresses: M rows of K codes and M fp32 scales."""
+    k = kernels
     M = x.shape[0]
-    packed_a, a_scale = quantized(M, K, x.device)
-    p = _lib.ptr
     if quant is k.swiglu_rot_quant_pack_a or quant is k.gate_rot_quant_pack_a:  # both operands at a pitch of K
         x, up = _dense(x), _dense(up)
-    else:
-        x = _rows(x)
+        _lib.check(quant(x.data_ptr(), up.data_ptr(), codes, scales, M, K, group, stream))
+        return
+    x = _rows(x)
     if quant is k.quant_pack_a:
-        launch(quant, M, 1, ROT_THREADS, [p(x), x.stride(0), p(packed_a), p(a_scale), M, K])
-    elif quant is k.swiglu_rot_quant_pack_a or quant is k.gate_rot_quant_pack_a:
-        launch(quant, M, 1, ROT_THREADS, [p(x), p(up), p(packed_a), p(a_scale), M, K, group])
+        _lib.check(quant(x.data_ptr(), x.stride(0), codes, scales, M, K, stream))
     else:
-        launch(quant, M, 1, ROT_THREADS, [p(x), x.stride(0), p(packed_a), p(a_scale), M, K, group])
-    return packed_a, a_scale
+        _lib.check(quant(x.data_ptr(), x.stride(0), codes, scales, M, K, group, stream))
+
+
+def _quantize_here(quant, x, K, up, group, stream):
+    """quantize() for a GEMM that follows at once: one workspace of M rows of K codes, then the M scales (16-byte aligned:
+    the entry points take K % 16 == 0). Returns (workspace, codes' address, scales' address)."""
+    M = x.shape[0]
+    workspace = torch.empty(M * (K + 4), dtype=torch.uint8, device=x.device)
+    codes = workspace.data_ptr()
+    _quantize_to(quant, x, K, up, group, codes, codes + M * K, stream)
+    return workspace, codes, codes + M * K
 
 
 def _check_linear(what, x, x_cols, K, weight, weight_dtypes, row_bytes, scales, n_scales, scales_dtype, bias, activations, up=None):
@@ -135,18 +149,21 @@ def _run(quant, gemm, x, weight, weight_scale, bias, K, up, activations, res, gr
     M = x.shape[0]
     N = weight.shape[0]
     out = torch.empty((M, N), dtype=torch.float16, device=x.device)
-    if out.numel() == 0:  # nothing to compute (the kernels reject empty shapes)
+    if M == 0 or N == 0:  # nothing to compute (the kernels reject empty shapes)
         return out
-    packed_a, a_scale = quantize(quant, x, K, up, group) if activations is None else activations
-    if res is not None:  # the epilogue reads the residual and its gate in 16-byte vectors
-        res = (_dense(res[0]), _dense(res[1]))
-    p = _lib.ptr
-    if gemm is k.gemm_i4:
-        launch(gemm, 0, 0, 0, [p(packed_a), p(weight), p(a_scale), p(weight_scale), p(bias), p(out), M, N, K])
+    stream = _lib.raw_stream()
+    if activations is None:
+        workspace, codes, scales = _quantize_here(quant, x, K, up, group, stream)
     else:
-        launch(gemm, 0, 0, 0, [p(packed_a), p(weight), p(a_scale), p(weight_scale), p(bias), p(out), M, N, K,
-                               p(res[0] if res is not None else None), p(res[1] if res is not None else None),
-                               res[0].shape[1] if res is not None else 1])
+        codes, scales = activations[0].data_ptr(), activations[1].data_ptr()
+    b = None if bias is None else bias.data_ptr()
+    if gemm is k.gemm_i4:
+        _lib.check(gemm(codes, weight.data_ptr(), scales, weight_scale.data_ptr(), b, out.data_ptr(), M, N, K, stream))
+    elif res is None:
+        _lib.check(gemm(codes, weight.data_ptr(), scales, weight_scale.data_ptr(), b, out.data_ptr(), M, N, K, None, None, 1, stream))
+    else:  # the epilogue reads the residual and its gate in 16-byte vectors
+        r, g = _dense(res[0]), _dense(res[1])
+        _lib.check(gemm(codes, weight.data_ptr(), scales, weight_scale.data_ptr(), b, out.data_ptr(), M, N, K, r.data_ptr(), g.data_ptr(), r.shape[1], stream))
     return out
 
 
@@ -186,15 +203,17 @@ def linear_w4a8(x, qweight, group_scales, bias=None, rotate=True, group=ROT_GROU
     if M == 0 or N == 0:
         return torch.empty((M, N), dtype=torch.float16, device=x.device)
     gemm = k.gemm_w4a8
+    stream = _lib.raw_stream()
     if activations is None:
+        quant = k.rot_quant_pack_a if rotate else k.quant_pack_a
         if _interleaved(qweight, group_scales, bias, N, K, rotate, scale_group):
-            activations, gemm = quantize(k.rot_quant_pack_a_il, x, K, None, group), k.gemm_w4a8_il
-        else:
-            activations = quantize(k.rot_quant_pack_a if rotate else k.quant_pack_a, x, K, None, group)
-    packed_a, a_scale = activations
+            quant, gemm = k.rot_quant_pack_a_il, k.gemm_w4a8_il
+        workspace, codes, scales = _quantize_here(quant, x, K, None, group, stream)
+    else:
+        codes, scales = activations[0].data_ptr(), activations[1].data_ptr()
     out = torch.empty((M, N), dtype=torch.float16, device=x.device)
-    p = _lib.ptr
-    launch(gemm, 0, 0, 0, [p(packed_a), p(qweight), p(a_scale), p(group_scales), p(bias), p(out), M, N, K, scale_group])
+    _lib.check(gemm(codes, qweight.data_ptr(), scales, group_scales.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(), M, N, K,
+                    scale_group, stream))
     return out
 
 
@@ -276,7 +295,9 @@ def wrap(original):
             return original(_replay_in_torch(x, rotate, situ, up), weight, weight_scale, bias, compute_dtype, x_q)
         N, K = weight.shape
         if isinstance(weight_scale, torch.Tensor) and weight_scale.numel() == N:
-            scale = weight_scale.reshape(N).float().contiguous()
+            scale = weight_scale
+            if scale.dim() != 1 or scale.dtype != torch.float32 or not scale.is_contiguous():
+                scale = scale.reshape(N).float().contiguous()
         else:
             scale = torch.full((N,), float(weight_scale), dtype=torch.float32, device=x.device)
         rows = x.reshape(-1, x.shape[-1]).contiguous()
@@ -349,9 +370,8 @@ def quantize_block_input(x, norm, scale, shift):
     x = _dense(x)  # read at a row pitch of K, in 16-byte vectors
     weight = _dense(comfy.model_management.cast_to(norm.scale, dtype=torch.float32, device=x.device))
     s, t = _dense(1 + scale), _dense(shift)
-    p = _lib.ptr
-    launch(get_kernels().mod_rot_quant_pack_a, B * L, 1, ROT_THREADS,
-           [p(x), p(packed_a), p(a_scale), B * L, K, p(weight), p(s), p(t), L, float(norm.eps)])
+    _lib.check(get_kernels().mod_rot_quant_pack_a(x.data_ptr(), packed_a.data_ptr(), a_scale.data_ptr(), B * L, K, weight.data_ptr(), s.data_ptr(),
+                                                  t.data_ptr(), L, float(norm.eps), _lib.raw_stream()))
     shared = packed_a, a_scale
 
 

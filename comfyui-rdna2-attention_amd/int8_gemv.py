@@ -15,7 +15,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib
-from .hip_attention import Kernels, launch
+from .hip_attention import Kernels
 
 try:  # The kernel wrappers work without ComfyUI; the patches below need it.
     import comfy_kitchen
@@ -69,7 +69,7 @@ def rotate(x, group):
         raise ValueError(f"rotate takes fp32 values in whole groups of {group}, not {x.numel()} of {x.dtype}")
     x = x.contiguous()
     rotated = torch.empty_like(x)
-    launch(get_kernels().rotate, x.numel() // group, 1, 256, [_lib.ptr(x), _lib.ptr(rotated), x.numel() // group, group])
+    _lib.check(get_kernels().rotate(x.data_ptr(), rotated.data_ptr(), x.numel() // group, group, _lib.raw_stream()))
     return rotated
 
 
@@ -101,8 +101,8 @@ def gemv(x, weight, scale, bias=None):
     N, K = weight.shape
     x = _row(x, K, (torch.float32, torch.float16), "gemv")
     out = torch.empty((*x.shape[:-1], N), dtype=x.dtype, device=x.device)
-    p = _lib.ptr
-    launch(get_kernels().gemv_i8, N // BLOCK_ROWS, 1, 256, [p(x), int(x.dtype == torch.float16), p(weight), p(scale), p(bias), p(out), N, K])
+    _lib.check(get_kernels().gemv_i8(x.data_ptr(), int(x.dtype == torch.float16), weight.data_ptr(), scale.data_ptr(),
+                                     None if bias is None else bias.data_ptr(), out.data_ptr(), N, K, _lib.raw_stream()))
     return out
 
 
@@ -123,8 +123,8 @@ def rotate_gemv(x, group, weight, scale, bias=None, rotated=None):
     x = _row(x, K, (torch.float32,), "rotate_gemv")
     rotated = _rotated_buffer(rotated, K)
     out = torch.empty((*x.shape[:-1], N), dtype=torch.float32, device=x.device)
-    p = _lib.ptr
-    launch(get_kernels().rotate_gemv_i8, N // BLOCK_ROWS, 1, 256, [p(x), group, p(weight), p(scale), p(bias), p(out), p(rotated), N, K])
+    _lib.check(get_kernels().rotate_gemv_i8(x.data_ptr(), group, weight.data_ptr(), scale.data_ptr(), None if bias is None else bias.data_ptr(),
+                                            out.data_ptr(), None if rotated is None else rotated.data_ptr(), N, K, _lib.raw_stream()))
     return out
 
 
@@ -302,7 +302,7 @@ def logits_gemv(x, weight):
     """fp32 logits (1, 1, N) of the last position of x (fp32) against a bf16 (N, K) table."""
     N, K = weight.shape
     out = torch.empty((1, 1, N), dtype=torch.float32, device=x.device)
-    launch(get_kernels().gemv_bf16, N // BLOCK_ROWS, 1, 256, [_lib.ptr(x), _lib.ptr(weight), _lib.ptr(out), N, K])
+    _lib.check(get_kernels().gemv_bf16(x.data_ptr(), weight.data_ptr(), out.data_ptr(), N, K, _lib.raw_stream()))
     return out
 
 
@@ -333,10 +333,10 @@ def attention_decode(q, k, v, lengths):
     out = torch.empty_like(q)
     partial = torch.empty((batch * heads, SPLITS, HEAD), dtype=torch.float32, device=q.device)
     stats = torch.empty((batch * heads, SPLITS, 2), dtype=torch.float32, device=q.device)
-    p = _lib.ptr
-    launch(k_.attn_decode, SPLITS, batch * kv_heads, 256, [p(q), p(k), p(v), p(lengths), p(partial), p(stats), batch, heads, kv_heads, capacity,
-                                                          HEAD ** -0.5])
-    launch(k_.attn_merge, batch * heads, 1, HEAD, [p(partial), p(stats), p(out), batch * heads])
+    stream = _lib.raw_stream()
+    _lib.check(k_.attn_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), lengths.data_ptr(), partial.data_ptr(), stats.data_ptr(), batch, heads, kv_heads,
+                              capacity, HEAD ** -0.5, stream))
+    _lib.check(k_.attn_merge(partial.data_ptr(), stats.data_ptr(), out.data_ptr(), batch * heads, stream))
     return out
 
 

@@ -5,7 +5,7 @@ import functools
 import torch
 
 from . import _lib
-from .hip_attention import Kernels, launch
+from .hip_attention import Kernels
 
 try:  # The kernel wrappers work without ComfyUI; forward() and patch() need it.
     import comfy.model_management
@@ -47,8 +47,7 @@ def rms_norm(x, weight, eps):
     if out.numel() == 0:  # nothing to compute (the kernels reject empty shapes)
         return out
     entry = k.rms_norm_head if D <= HEAD_DIM else k.rms_norm_row
-    p = _lib.ptr
-    launch(entry, 0, 0, THREADS, [p(x), p(weight), p(out), B, H, L, D, sb, sh, sl, float(eps)])
+    _lib.check(entry(x.data_ptr(), weight.data_ptr(), out.data_ptr(), B, H, L, D, sb, sh, sl, float(eps), _lib.raw_stream()))
     return out
 
 
@@ -67,9 +66,8 @@ def rms_norm_rope(x, heads, module, freqs):
     if weight.numel() != HEAD_DIM or not weight.is_contiguous():
         raise ValueError(f"rms_norm_rope takes {HEAD_DIM} norm weights")
     batch_stride = L * HEAD_DIM // 2 if freqs.shape[0] > 1 else 0
-    p = _lib.ptr
-    launch(get_kernels().rms_norm_rope, 0, 0, THREADS, [p(x), p(weight), p(out), B, heads, L, HEAD_DIM, x.stride(0), HEAD_DIM, x.stride(1),
-                                                        float(module.eps), p(freqs), batch_stride])
+    _lib.check(get_kernels().rms_norm_rope(x.data_ptr(), weight.data_ptr(), out.data_ptr(), B, heads, L, HEAD_DIM, x.stride(0), HEAD_DIM, x.stride(1),
+                                           float(module.eps), freqs.data_ptr(), batch_stride, _lib.raw_stream()))
     return out
 
 
