@@ -91,6 +91,29 @@ def test_gate_every_fp16_gate(dev):
     assert_same(q_of(packed, M, K), q_ref)
 
 
+# Waves per row and passes: 2 waves for five groups; 5 and 6 waves, the last pass partly empty; past 6144 values 4 waves (six
+# below 1024 rows), with two and three passes.
+@pytest.mark.parametrize("act", ["rot", "swiglu", "gate"])
+@pytest.mark.parametrize("M,K,group", [(9, 1280, 256), (5, 4608, 256), (7, 5376, 128), (3, 6400, 256), (1025, 6400, 128), (1024, 12544, 256), (2, 12544, 128)])
+def test_rot_quant_wave_counts_bit_exact(dev, act, M, K, group):
+    """Gates span +-4.2, so that lanes take either of the fast sigmoid's two error bounds."""
+    print(f"wave counts {act} M={M} K={K} group={group}", flush=True)
+    g, k = gen(K + M), kern()
+    x, u = torch.randn(M, K, generator=g).half(), torch.randn(M, K, generator=g).half()
+    gates = (torch.rand(M, K, generator=g) * 8.4 - 4.2).half()
+    if act == "rot":
+        packed, scale = int8_gemm.quantize(k.rot_quant_pack_a, x.to(dev), K, group=group)
+        q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), group=group)
+    elif act == "swiglu":
+        packed, scale = int8_gemm.quantize(k.swiglu_rot_quant_pack_a, gates.to(dev), K, up=u.to(dev), group=group)
+        q_ref, s_ref, _ = oracle.rot_quant_rows(gates.numpy(), act=oracle.ACT_SWIGLU, group=group, u=u.numpy())
+    else:
+        packed, scale = int8_gemm.quantize(k.gate_rot_quant_pack_a, x.to(dev), K, up=gates.to(dev), group=group)
+        q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), act=oracle.ACT_GATE, group=group, u=gates.numpy())
+    assert_same(scale.cpu().numpy(), s_ref)
+    assert_same(q_of(packed, M, K), q_ref)
+
+
 @pytest.mark.parametrize("B,L,K", [(1, 77, 3072), (2, 40, 1024)])
 def test_mod_rot_quant_bit_exact(dev, B, L, K):
     print(f"mod_rot_quant B={B} L={L} K={K}", flush=True)
