@@ -458,22 +458,17 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
     // Copy instruction j of a wave fills rows (4 j + wave) RPI .. + RPI - 1 of A (or of W, with RPIB): lane i
     // takes row (4 j + wave) RPI + i / CPR at physical chunk i % CPR, i.e. logical chunk cchunk (the swizzle
     // term is the same for every j). A rows past M re-read row M - 1 and W rows past N row N - 1 (their results
-    // are not stored); the clamp is folded into the per-lane offsets, taken from a clamped group base so that they
-    // are never negative (they are the unsigned 32-bit voffset of the copy).
+    // are not stored). The rows' offsets from the tile's first one are per lane (the unsigned 32-bit voffset of the
+    // copy: 256 rows of K < 2^24 bytes), so that all of a slice's copies share one scalar address per operand.
     const int crow = wave * RPI + lane / CPR, cchunk = (lane % CPR) ^ ((crow / RPL) % CPR);
     const int brow = wave * RPIB + lane / CPRB, bchunk = (lane % CPRB) ^ ((brow / RPLB) % CPRB);
-    int arow[AI], wrow0[BI];
     u32 aoff[AI], boff[BI];
+    const int8_t* const abase = A + (size_t)m0 * K;  // the tile's first row and first column exist: m0 < M, n0 < N
+    const int8_t* const wbase = W + (size_t)n0 * wrow;
 #pragma unroll
-    for (int c = 0; c < AI; c++) {
-        arow[c] = min(m0 + NW * RPI * c, M - 1);
-        aoff[c] = (u32)(min(m0 + NW * RPI * c + crow, M - 1) - arow[c]) * K + cchunk * 16;
-    }
+    for (int c = 0; c < AI; c++) aoff[c] = (u32)min(NW * RPI * c + crow, M - 1 - m0) * K + cchunk * 16;
 #pragma unroll
-    for (int c = 0; c < BI; c++) {
-        wrow0[c] = min(n0 + NW * RPIB * c, N - 1);
-        boff[c] = (u32)(min(n0 + NW * RPIB * c + brow, N - 1) - wrow0[c]) * wrow + bchunk * 16;
-    }
+    for (int c = 0; c < BI; c++) boff[c] = (u32)min(NW * RPIB * c + brow, N - 1 - n0) * wrow + bchunk * 16;
     auto stage = [&](int kt) -> const char* { return smem + (kt % NS) * STAGE; };
     // The epilogue's scales go to a scale block: ws[n0 .. n0 + BN) (BN / 64 copies of 64 floats; those past N, a
     // multiple of 64, re-read the first), bias[n0 ..) (256-byte copies, lanes past BN / 2 or N / 2 re-read the last
@@ -516,8 +511,8 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
     }
     auto copy = [&](int kt, int c) {  // copy instruction c (< NI) of slice kt
         const char* st = stage(kt);
-        if (c < AI) dma16(A + (size_t)arow[c] * K + kt * KB8, aoff[c], st + (NW * c + wave) * 1024);
-        else dma16(W + (size_t)wrow0[c - AI] * wrow + kt * WB, boff[c - AI], st + BM * KB8 + (NW * (c - AI) + wave) * 1024);
+        if (c < AI) dma16(abase + (size_t)kt * KB8, aoff[c], st + (NW * c + wave) * 1024);
+        else dma16(wbase + (size_t)kt * WB, boff[c - AI], st + BM * KB8 + (NW * (c - AI) + wave) * 1024);
     };
 
     // Fragment f (< FI: A block f, else W block f - FI) of k step kk: row base + lq, k values 32 kk + 16 g ..
@@ -904,7 +899,7 @@ static int narrow_slice_width(int M, int N) {
 template <bool W4, int EPI, bool IL = false>
 static int dispatch8(const void* a, const void* w, const float* as, const float* ws, const void* gs, const void* bias, void* c, int M, int N, int K,
                      int group, const void* R, const void* G, int L, void* stream) {
-    if (K >= (1 << 24)) return -1;  // per-lane copy offsets (< 64 K) must fit the 32-bit voffset
+    if (K >= (1 << 24)) return -1;  // per-lane copy offsets (< 256 K) must fit the 32-bit voffset
     if (W4 && K > 65536) return -1;  // 16 x the int4 products, summed over K, must fit in int32
     // The row-segment epilogue reads ws as float4 and bias / R / G and writes C as 8-byte (int32: 16-byte) vectors.
     auto aligned = [](const void* p, uintptr_t al) { return ((uintptr_t)p & (al - 1)) == 0; };
