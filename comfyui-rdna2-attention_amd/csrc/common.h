@@ -114,7 +114,7 @@ __device__ __forceinline__ i4v as_i4(u4v v) { return __builtin_bit_cast(i4v, v);
 // Cross-lane reductions on DPP and lane-swap instructions (one VALU op per step, no LDS round trip).
 // Every lane of a group receives the same bits: partners always add the same two partial values.
 template <int CTRL>
-__device__ __forceinline__ float dpp(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false)); }
+__device__ __forceinline__ float dpp(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true)); }
 // Over the 16 lanes of each row (lanes 16 r .. 16 r + 15): xor 1, xor 2 (quad_perm), then the half-row
 // mirror (i <-> 7 - i) and the row mirror (i <-> 15 - i).
 __device__ __forceinline__ float row_sum16(float x) {

@@ -7,14 +7,15 @@
 // and, for TPR 256, the eight half-wave sums are added in order. rstd = 1 / sqrt(sum / D + eps)
 // (correctly rounded, where the reference has rsqrtf), y = fp16(x * rstd * (w + 1)).
 // Rows are addressed with (b, h, l) strides, so Q and K are read straight from a linear output;
-// the result is written contiguous (B, H, L, D).
+// the result is written contiguous (B, H, L, D). norm_kernel does a row per TPR threads; norm_rope_kernel, whose
+// rows have D = 128, one or two heads of a token per 16 threads.
 #include "common.h"
 
 #define NT 256
 
-template <int TPR, int CHUNKS, bool ROPE>
+template <int TPR, int CHUNKS>
 __global__ __launch_bounds__(NT) void norm_kernel(const half_t* __restrict__ X, const float* __restrict__ W, half_t* __restrict__ Y, int rows, int D, int L,
-                                                  int H, long sb, long sh, long sl, float eps, const f4* __restrict__ F, long fb) {
+                                                  int H, long sb, long sh, long sl, float eps) {
     __shared__ float red[NT / 32];
     const int t = threadIdx.x % TPR, n = blockIdx.x * (NT / TPR) + threadIdx.x / TPR;
     if (TPR < NT && n >= rows) return;
@@ -64,21 +65,52 @@ __global__ __launch_bounds__(NT) void norm_kernel(const half_t* __restrict__ X, 
             h8 o;
 #pragma unroll
             for (int j = 0; j < 8; j++) o[j] = to_half((float)v[c][j] * rstd * ((j < 4 ? lo[j & 3] : hi[j & 3]) + 1.f));
-            if (ROPE) {
-                // rms_norm.hip:48-61: a = fma(m1, x1, fp32(m0 x0)), c = fma(m3, x1, fp32(m2 x0)), each
-                // rounded to fp32 and then to fp16 (to_half), like the reference.
-                const f4* f = F + b * fb + (long)l * (D / 2) + i * 4;
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const f4 m = f[j];
-                    const float x0 = (float)o[j * 2], x1 = (float)o[j * 2 + 1];
-                    const float a = __builtin_fmaf(m[1], x1, m[0] * x0), cc = __builtin_fmaf(m[3], x1, m[2] * x0);
-                    o[j * 2] = to_half(a);
-                    o[j * 2 + 1] = to_half(cc);
-                }
-            }
             y[i] = o;
         }
+    }
+}
+
+// HPT heads of one token per 16 threads, H / HPT apart so that neighbouring slots still read neighbouring rows. What bounds
+// a row of one head is not its 512 bytes of x and y but the 1.5 KiB of weight and frequencies each head's threads load
+// again from L2; two heads share them. 4096 x 24 heads 13.2 -> 11.5 us (4.4 TB/s of x, y), 8192 x 24 22.3 -> 19.0; four
+// heads measured 11.3 and 19.5.
+template <int HPT>
+__global__ __launch_bounds__(NT) void norm_rope_kernel(const half_t* __restrict__ X, const float* __restrict__ W, half_t* __restrict__ Y, int units, int L, int H,
+                                                       long sb, long sh, long sl, float eps, const f4* __restrict__ F, long fb) {
+    constexpr int D = 128, TPR = 16;
+    const int t = threadIdx.x % TPR, n = blockIdx.x * (NT / TPR) + threadIdx.x / TPR;
+    if (n >= units) return;
+    const int G = H / HPT, h0 = n % G, l = (n / G) % L, b = n / G / L;
+    const half_t* x = X + b * sb + l * sl + t * 8;
+    // Every load up front, as in norm_kernel.
+    h8 v[HPT];
+    f4 m[4];
+#pragma unroll
+    for (int c = 0; c < HPT; c++) v[c] = *(const h8*)(x + (h0 + c * G) * sh);
+    const f4 lo = ((const f4*)W)[t * 2], hi = ((const f4*)W)[t * 2 + 1];
+    const f4* f = F + b * fb + (long)l * (D / 2) + t * 4;
+#pragma unroll
+    for (int j = 0; j < 4; j++) m[j] = f[j];
+#pragma unroll
+    for (int c = 0; c < HPT; c++) {
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) sum = __builtin_fmaf((float)v[c][j], (float)v[c][j], sum);
+        sum = xor_butterfly_sum<16>(sum);
+        const float rstd = 1.f / sqrtf(sum / (float)D + eps);
+        h8 o;
+#pragma unroll
+        for (int j = 0; j < 8; j++) o[j] = to_half((float)v[c][j] * rstd * ((j < 4 ? lo[j & 3] : hi[j & 3]) + 1.f));
+        // rms_norm.hip:48-61: a = fma(m1, x1, fp32(m0 x0)), c = fma(m3, x1, fp32(m2 x0)), each rounded to fp32 and then to
+        // fp16 (to_half), like the reference.
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float x0 = (float)o[j * 2], x1 = (float)o[j * 2 + 1];
+            const float a = __builtin_fmaf(m[j][1], x1, m[j][0] * x0), d = __builtin_fmaf(m[j][3], x1, m[j][2] * x0);
+            o[j * 2] = to_half(a);
+            o[j * 2 + 1] = to_half(d);
+        }
+        *(h8*)(Y + ((size_t)(b * H + h0 + c * G) * L + l) * D + t * 8) = o;
     }
 }
 
@@ -90,8 +122,8 @@ extern "C" {
 int rda_rms_norm_head(const void* x, const float* w, void* y, int B, int H, int L, int D, long sb, long sh, long sl, float eps, void* stream) {
     if (!norm_ok(B, H, L, D) || D > 128) return RDA_ERR_INVALID;
     const int rows = B * H * L;
-    hipLaunchKernelGGL((norm_kernel<16, 1, false>), dim3((rows + 15) / 16), dim3(NT), 0, (hipStream_t)stream, (const half_t*)x, w, (half_t*)y, rows, D, L,
-                       H, sb, sh, sl, eps, nullptr, 0L);
+    hipLaunchKernelGGL((norm_kernel<16, 1>), dim3((rows + 15) / 16), dim3(NT), 0, (hipStream_t)stream, (const half_t*)x, w, (half_t*)y, rows, D, L,
+                       H, sb, sh, sl, eps);
     return (int)hipGetLastError();
 }
 
@@ -101,15 +133,14 @@ int rda_rms_norm_row(const void* x, const float* w, void* y, int B, int H, int L
     const int rows = B * H * L;
     // Chunks per thread: as many as D needs (the loads of a thread's unused chunks are not free).
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(rows), dim3(NT), 0, (hipStream_t)stream, (const half_t*)x, w, (half_t*)y, rows, D, L, H, sb, sh, sl, eps, nullptr,
-                           0L);
+        hipLaunchKernelGGL(kern, dim3(rows), dim3(NT), 0, (hipStream_t)stream, (const half_t*)x, w, (half_t*)y, rows, D, L, H, sb, sh, sl, eps);
         return (int)hipGetLastError();
     };
     switch ((D / 8 + NT - 1) / NT) {
-    case 1: return launch(norm_kernel<NT, 1, false>);
-    case 2: return launch(norm_kernel<NT, 2, false>);
-    case 3: return launch(norm_kernel<NT, 3, false>);
-    default: return launch(norm_kernel<NT, 4, false>);
+    case 1: return launch(norm_kernel<NT, 1>);
+    case 2: return launch(norm_kernel<NT, 2>);
+    case 3: return launch(norm_kernel<NT, 3>);
+    default: return launch(norm_kernel<NT, 4>);
     }
 }
 
@@ -119,9 +150,15 @@ int rda_rms_norm_rope(const void* x, const float* w, void* y, int B, int H, int 
                       long fb, void* stream) {
     if (!norm_ok(B, H, L, D) || D != 128) return RDA_ERR_INVALID;
     const int rows = B * H * L;
-    hipLaunchKernelGGL((norm_kernel<16, 1, true>), dim3((rows + 15) / 16), dim3(NT), 0, (hipStream_t)stream, (const half_t*)x, w, (half_t*)y, rows, D, L,
-                       H, sb, sh, sl, eps, (const f4*)freqs, fb);
-    return (int)hipGetLastError();
+    auto launch = [&](auto kern, int units) {
+        hipLaunchKernelGGL(kern, dim3((units + 15) / 16), dim3(NT), 0, (hipStream_t)stream, (const half_t*)x, w, (half_t*)y, units, L, H, sb, sh, sl, eps,
+                           (const f4*)freqs, fb);
+        return (int)hipGetLastError();
+    };
+    // Two heads per slot need twice the rows to fill the chip: at 12288 rows both take 3.6 us, at 26424 one head per slot
+    // takes 5.35 and two 5.1, at 2100 2.2 and 2.5. An odd number of heads stays with one.
+    if (H % 2 == 0 && rows >= 16384) return launch(norm_rope_kernel<2>, rows / 2);
+    return launch(norm_rope_kernel<1>, rows);
 }
 
 int rda_version(void) { return 1; }

@@ -270,6 +270,20 @@ def test_rms_norm_rope_bit_exact(dev, fb):
     assert_same(bits(out), bits(ref))
 
 
+@pytest.mark.parametrize("B,L,H", [(1, 8191, 2), (1, 8192, 2), (1, 8192, 3), (2, 683, 12), (3, 911, 6), (1, 1025, 16)])
+def test_rms_norm_rope_heads_per_slot_bit_exact(dev, B, L, H):
+    """Either side of 16384 rows, where an even number of heads goes two to a slot; the last workgroup partly empty."""
+    print(f"rms_norm_rope slots B={B} L={L} H={H}", flush=True)
+    g = gen(L + H)
+    fused = torch.randn(B, L, 2 * H * 128, generator=g).half()
+    w = (torch.randn(128, generator=g) * 0.1).float()
+    ang = torch.randn(B, 1, L, 64, generator=g)
+    freqs = torch.stack([torch.cos(ang), -torch.sin(ang), torch.sin(ang), torch.cos(ang)], -1).reshape(B, 1, L, 64, 2, 2).float()
+    out = rms_norm.rms_norm_rope(fused.to(dev)[:, :, H * 128:], H, _Norm(w.to(dev), 1e-6), freqs.to(dev))
+    xh = fused[:, :, H * 128:].reshape(B, L, H, 128).transpose(1, 2).contiguous().numpy()
+    assert_same(bits(out), bits(oracle.rms_norm(xh, w.numpy(), 1e-6, freqs=freqs.numpy())))
+
+
 @pytest.mark.parametrize("seed", range(10))
 def test_norms_random_shapes(dev, seed):
     """Seeded random shapes, bit for bit against the oracle: RMSNorm of (B, L, D) or (B, H, L, D) (up to 1 x 600, 4 x 300,
