@@ -59,6 +59,10 @@ __device__ __forceinline__ h2 to_half2(float a, float b) {
     asm("" : "+v"(a), "+v"(b));  // round to fp32 first, as in to_half
     return __builtin_convertvector((f2){a, b}, h2);
 }
+// a * s + c in fp32 for the low (HI false) or high fp16 value a of a word: the compiler makes it one mixed-precision FMA
+// (v_fma_mix_f32), without a conversion. With c = 0 it is the fp32 product, up to the sign of a zero, which no code depends on.
+template <bool HI>
+__device__ __forceinline__ float mix(u32 w, float s, float c = 0.f) { return __builtin_fmaf((float)__builtin_bit_cast(h2, w)[HI], s, c); }
 // SwiGLU (int8_gemm.hip:130-132): r16(r16(silu(g)) u) with silu(g) = g / (1 + rda_expf(-g)) in fp32; the sigmoid
 // gate (int8_gemm.hip:135-137): r16(x r16(sigmoid(gate))), sigmoid(g) = 1 / (1 + rda_expf(-g)) in fp32.
 // Both take a fast path -- hardware exp2 of a rounded argument and a hardware reciprocal -- whose value q lies
@@ -69,9 +73,11 @@ __device__ __forceinline__ h2 to_half2(float a, float b) {
 // and at the overflow threshold too, and values too small for fp32's normal range round to zero either way. The
 // pairs where the ends differ (about 0.3% of values) take the exact formula; the SwiGLU and gate tests run every
 // finite fp16 gate through the kernels and compare the codes, which then fix r16 of the value, with the oracle's.
-__device__ __forceinline__ float silu_fast(float g) { return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-g * 1.44269504088896341f)); }
+template <bool HI>
+__device__ __forceinline__ float sigmoid_fast(u32 g) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(mix<HI>(g, -1.44269504088896341f))); }
+template <bool HI>
+__device__ __forceinline__ float silu_fast(u32 g) { return mix<HI>(g, sigmoid_fast<HI>(g)); }
 __device__ __forceinline__ float silu_exact(float g) { return g / (1.f + rda_expf(-g)); }
-__device__ __forceinline__ float sigmoid_fast(float g) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-g * 1.44269504088896341f)); }
 __device__ __forceinline__ float sigmoid_exact(float g) { return 1.f / (1.f + rda_expf(-g)); }
 // For |g| < 4 q lies within 2.3 x 2^-23 of the exact value, relatively (measured on every such gate), so a lane whose 16
 // gates all do, as nearly all of a model's, takes d = 3 x 2^-23 (half an ulp of the ends' own rounding included) and the
@@ -114,10 +120,10 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// (int)floorf(x) in one instruction (the compiler emits a floor and a truncation); x is finite here.
-__device__ __forceinline__ int cvt_floor(float x) {
+// (int)floorf(x + 0.5f) in one instruction; x is finite here.
+__device__ __forceinline__ int cvt_nearest_up(float x) {
     int r;
-    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
     return r;
 }
 
@@ -129,7 +135,9 @@ __device__ __forceinline__ u32 pack4(int a, int b, int c, int d) {
 
 // GROUP 256 or 128 rotates; GROUP 0 is quant_pack_a (no rotation, int8_gemm.hip:93-103). NW waves per row: the
 // launcher sizes it to the row (launch_rot_quant; K = 3072 keeps every lane of three waves busy in both passes: the kernel
-// is vector-ALU bound); MOD keeps 4 (QT threads), whose sum of squares follows the reference's thread order.
+// is vector-ALU bound: 306 instructions per wave and 1024 values, 112 of them the butterflies, 411 before the conversions
+// were folded into multiply-adds: 4096 x 3072 10.8 -> 9.6 us (3.9 TB/s), SwiGLU 4096 x 8192 36.2 -> 34.0, MOD 4096 x 3072
+// 17.8 -> 15.8); MOD keeps 4 (QT threads), whose sum of squares follows the reference's thread order.
 // IL: the codes k-interleaved (each 8 values of k stored as their 4 even ones, then their 4 odd ones).
 // WL (the rotations other than MOD): each wave keeps the rotated fp16 values of its own passes (1024 values each) in an
 // LDS region of its own -- pass p at SW_BYTES + 2048 p, the last pass inside its transpose buffer, free by then -- and
@@ -139,6 +147,19 @@ __device__ __forceinline__ u32 pack4(int a, int b, int c, int d) {
 #define SW_BYTES (64 * 17 * 4)  // a wave's transpose buffer: 17 floats per lane
 template <int GROUP, int NW>
 __host__ __device__ constexpr int rot_passes(int K) { return (K / GROUP + NW * (1024 / GROUP) - 1) / (NW * (1024 / GROUP)); }
+
+// The wave's maximum of values >= 0, none NaN: they order as their bits do, and an integer maximum needs no canonical inputs.
+__device__ __forceinline__ float wave_max(float x) {
+    u32 m = __float_as_uint(x);
+    m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xF, 0xF, true));
+    m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xF, 0xF, true));
+    m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xF, 0xF, true));
+    m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x140, 0xF, 0xF, true));
+    const auto a = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+    m = max(a[0], a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+    return __uint_as_float(max(b[0], b[1]));
+}
 
 template <int ACT, bool I4, int GROUP, int NW, bool IL>
 __global__ __launch_bounds__(NW * 64) void rot_quant_kernel(const half_t* __restrict__ X, long ldx, const half_t* __restrict__ U,
@@ -196,120 +217,126 @@ __global__ __launch_bounds__(NW * 64) void rot_quant_kernel(const half_t* __rest
         const size_t mrow = ACT == MOD ? (size_t)(row / mod.L) * K : 0;
         const half_t* ms = ACT == MOD ? mod.s + mrow : nullptr;
         const half_t* mt = ACT == MOD ? mod.t + mrow : nullptr;
-        const float norm = GROUP == 256 ? 0.0625f : 0.0883883461356163025f;
+        // A group of 256 is scaled by 1/16, a power of two: applied to the fp16 inputs in the conversion (exact, and every sum
+        // then rounds as the unscaled one does; nothing is near fp32's subnormals) it costs no instruction, and the rotated
+        // values convert to fp16 in pairs. A group of 128 is scaled after its rotation, rounded to fp32 first.
+        constexpr float pre = GROUP == 256 ? 0.0625f : 1.f, norm = GROUP == 256 ? 1.f : 0.0883883461356163025f;
+        auto widen = [&](h2 p, float& a, float& b) __attribute__((always_inline)) {
+            const u32 w = __builtin_bit_cast(u32, p);
+            a = pre != 1.f ? mix<false>(w, pre) : (float)p[0];
+            b = pre != 1.f ? mix<true>(w, pre) : (float)p[1];
+        };
 
         for (int g0 = wave * GPW; g0 < groups; g0 += NW * GPW) {
-            const int g = g0 + gl;
-            const bool active = g < groups;
+            // Lanes past the row's groups redo its last one (their results are not kept): no branch around the work.
+            const bool active = g0 + gl < groups;
+            const int g = active ? g0 + gl : groups - 1;
             float v[16];
-            if (active) {
-                const int e0 = g * GROUP + c * 16;
-                const half_t* src = ACT == MOD ? rotated : x;
-                const h8 lo = *(const h8*)(src + e0), hi = *(const h8*)(src + e0 + 8);
-                if (ACT == SITU) {
-                    const h8 glo = *(const h8*)(x + K + e0), ghi = *(const h8*)(x + K + e0 + 8);
+            const int e0 = g * GROUP + c * 16;
+            const half_t* src = ACT == MOD ? rotated : x;
+            const h8 lo = *(const h8*)(src + e0), hi = *(const h8*)(src + e0 + 8);
+            if (ACT == SITU) {
+                const h8 glo = *(const h8*)(x + K + e0), ghi = *(const h8*)(x + K + e0 + 8);
 #pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        v[i] = situ((float)lo[i], (float)glo[i]);
-                        v[8 + i] = situ((float)hi[i], (float)ghi[i]);
-                    }
-                } else if (ACT == SWIGLU) {
-                    const half_t* u = U + (size_t)row * K;
-                    const h8 ulo = *(const h8*)(u + e0), uhi = *(const h8*)(u + e0 + 8);
-                    const Sure sure = sure_of(lo, hi);
-#pragma unroll
-                    for (int i = 0; i < 16; i += 2) {
-                        const float g0 = (float)(i < 8 ? lo[i] : hi[i - 8]), g1 = (float)(i < 8 ? lo[i + 1] : hi[i - 7]);
-                        const h2 sg = round_sure(silu_fast(g0), silu_fast(g1), sure, [&](int k) { return silu_exact(k ? g1 : g0); });
-                        const h2 pr = sg * (h2){i < 8 ? ulo[i] : uhi[i - 8], i < 8 ? ulo[i + 1] : uhi[i - 7]};
-                        v[i] = (float)pr[0];
-                        v[i + 1] = (float)pr[1];
-                    }
-                } else if (ACT == GATE) {
-                    const half_t* u = U + (size_t)row * K;
-                    const h8 ulo = *(const h8*)(u + e0), uhi = *(const h8*)(u + e0 + 8);
-                    const Sure sure = sure_of(ulo, uhi);
-#pragma unroll
-                    for (int i = 0; i < 16; i += 2) {
-                        const float g0 = (float)(i < 8 ? ulo[i] : uhi[i - 8]), g1 = (float)(i < 8 ? ulo[i + 1] : uhi[i - 7]);
-                        const h2 sg = round_sure(sigmoid_fast(g0), sigmoid_fast(g1), sure, [&](int k) { return sigmoid_exact(k ? g1 : g0); });
-                        const h2 pr = (h2){i < 8 ? lo[i] : hi[i - 8], i < 8 ? lo[i + 1] : hi[i - 7]} * sg;
-                        v[i] = (float)pr[0];
-                        v[i + 1] = (float)pr[1];
-                    }
-                } else if (ACT == MOD) {
-                    const h8 slo = *(const h8*)(ms + e0), shi = *(const h8*)(ms + e0 + 8);
-                    const h8 tlo = *(const h8*)(mt + e0), thi = *(const h8*)(mt + e0 + 8);
-                    const f4* w = (const f4*)(mod.w + e0);
-                    const f4 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
-                    const float wv[16] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w, w3.x, w3.y, w3.z, w3.w};
-#pragma unroll
-                    for (int i = 0; i < 16; i += 2) {
-                        // modulate (int8_gemm.hip:140-143): r16(r16(r16(x rstd (w + 1)) s) + t), two elements at a time.
-                        const h8 &xs = i < 8 ? lo : hi, &ss = i < 8 ? slo : shi, &ts = i < 8 ? tlo : thi;
-                        const int j = i & 7;
-                        const h2 a = to_half2((float)xs[j] * rstd * (wv[i] + 1.f), (float)xs[j + 1] * rstd * (wv[i + 1] + 1.f));
-                        const h2 m = a * (h2){ss[j], ss[j + 1]} + (h2){ts[j], ts[j + 1]};
-                        v[i] = (float)m[0];
-                        v[i + 1] = (float)m[1];
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        v[i] = (float)lo[i];
-                        v[8 + i] = (float)hi[i];
-                    }
+                for (int i = 0; i < 8; i++) {
+                    v[i] = situ((float)lo[i], (float)glo[i]) * pre;
+                    v[8 + i] = situ((float)hi[i], (float)ghi[i]) * pre;
                 }
-                h16(v);  // digits at strides 1 and 4
+            } else if (ACT == SWIGLU) {
+                const half_t* u = U + (size_t)row * K;
+                const h8 ulo = *(const h8*)(u + e0), uhi = *(const h8*)(u + e0 + 8);
+                const Sure sure = sure_of(lo, hi);
 #pragma unroll
-                for (int i = 0; i < 16; i++) sw[c * 17 + i] = v[i];
+                for (int i = 0; i < 16; i += 2) {
+                    const h2 g = {i < 8 ? lo[i] : hi[i - 8], i < 8 ? lo[i + 1] : hi[i - 7]};
+                    const u32 w = __builtin_bit_cast(u32, g);
+                    const h2 sg = round_sure(silu_fast<false>(w), silu_fast<true>(w), sure, [&](int k) { return silu_exact((float)g[k]); });
+                    const h2 pr = sg * (h2){i < 8 ? ulo[i] : uhi[i - 8], i < 8 ? ulo[i + 1] : uhi[i - 7]};
+                    widen(pr, v[i], v[i + 1]);
+                }
+            } else if (ACT == GATE) {
+                const half_t* u = U + (size_t)row * K;
+                const h8 ulo = *(const h8*)(u + e0), uhi = *(const h8*)(u + e0 + 8);
+                const Sure sure = sure_of(ulo, uhi);
+#pragma unroll
+                for (int i = 0; i < 16; i += 2) {
+                    const h2 g = {i < 8 ? ulo[i] : uhi[i - 8], i < 8 ? ulo[i + 1] : uhi[i - 7]};
+                    const u32 w = __builtin_bit_cast(u32, g);
+                    const h2 sg = round_sure(sigmoid_fast<false>(w), sigmoid_fast<true>(w), sure, [&](int k) { return sigmoid_exact((float)g[k]); });
+                    const h2 pr = (h2){i < 8 ? lo[i] : hi[i - 8], i < 8 ? lo[i + 1] : hi[i - 7]} * sg;
+                    widen(pr, v[i], v[i + 1]);
+                }
+            } else if (ACT == MOD) {
+                const h8 slo = *(const h8*)(ms + e0), shi = *(const h8*)(ms + e0 + 8);
+                const h8 tlo = *(const h8*)(mt + e0), thi = *(const h8*)(mt + e0 + 8);
+                const f4* w = (const f4*)(mod.w + e0);
+                const f4 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
+                const float wv[16] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w, w3.x, w3.y, w3.z, w3.w};
+#pragma unroll
+                for (int i = 0; i < 16; i += 2) {
+                    // modulate (int8_gemm.hip:140-143): r16(r16(r16(x rstd (w + 1)) s) + t), two elements at a time.
+                    const h8 &xs = i < 8 ? lo : hi, &ss = i < 8 ? slo : shi, &ts = i < 8 ? tlo : thi;
+                    const int j = i & 7;
+                    const u32 xw = __builtin_bit_cast(u32, (h2){xs[j], xs[j + 1]});
+                    const h2 a = to_half2(mix<false>(xw, rstd) * (wv[i] + 1.f), mix<true>(xw, rstd) * (wv[i + 1] + 1.f));
+                    const h2 m = a * (h2){ss[j], ss[j + 1]} + (h2){ts[j], ts[j + 1]};
+                    widen(m, v[i], v[i + 1]);
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; i += 2) {
+                    widen((h2){lo[i], lo[i + 1]}, v[i], v[i + 1]);
+                    widen((h2){hi[i], hi[i + 1]}, v[8 + i], v[8 + i + 1]);
+                }
             }
+            h16(v);  // digits at strides 1 and 4
+#pragma unroll
+            for (int i = 0; i < 16; i++) sw[c * 17 + i] = v[i];
             wave_sync();
-            if (active) {
-                if (GROUP == 256) {
-                    // Lane c now holds elements c + 16i: digits at strides 16 and 64.
+            if (GROUP == 256) {
+                // Lane c now holds elements c + 16i: digits at strides 16 and 64.
 #pragma unroll
-                    for (int i = 0; i < 16; i++) v[i] = sw[i * 17 + c];
-                    h16(v);
-                } else {
-                    // Lane c takes the columns c and c + 8 (elements c + 16i, c + 8 + 16i, i < 8):
-                    // an H4 over the stride-16 digit, then an H2 over the stride-64 digit.
+                for (int i = 0; i < 16; i++) v[i] = sw[i * 17 + c];
+                h16(v);
+            } else {
+                // Lane c takes the columns c and c + 8 (elements c + 16i, c + 8 + 16i, i < 8):
+                // an H4 over the stride-16 digit, then an H2 over the stride-64 digit.
 #pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        v[i] = sw[i * 17 + c];
-                        v[8 + i] = sw[i * 17 + c + 8];
-                    }
-#pragma unroll
-                    for (int b = 0; b < 16; b += 4) h4(v[b], v[b + 1], v[b + 2], v[b + 3]);
-#pragma unroll
-                    for (int b = 0; b < 16; b += 8)
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const float p = v[b + i], q = v[b + i + 4];
-                            v[b + i] = p + q;
-                            v[b + i + 4] = p - q;
-                        }
+                for (int i = 0; i < 8; i++) {
+                    v[i] = sw[i * 17 + c];
+                    v[8 + i] = sw[i * 17 + c + 8];
                 }
+#pragma unroll
+                for (int b = 0; b < 16; b += 4) h4(v[b], v[b + 1], v[b + 2], v[b + 3]);
+#pragma unroll
+                for (int b = 0; b < 16; b += 8)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float p = v[b + i], q = v[b + i + 4];
+                        v[b + i] = p + q;
+                        v[b + i + 4] = p - q;
+                    }
             }
             // The row maximum is taken before the rounding to fp16 and rounded once at the end: rounding is monotonic,
             // so max(round |p|) = round(max |p|), one conversion per element fewer.
             const int p = (g0 - wave * GPW) / (NW * GPW);
             if (WL && p == passes - 1) wave_sync();  // the last pass reuses the transpose buffer: every lane has read it
-            if (active) {
+            if (WL || active) {
                 half_t* dst = WL ? (half_t*)(wbase + (p == passes - 1 ? 0 : SW_BYTES + 2048 * p)) + gl * GROUP : rotated + g * GROUP;
 #pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const float y = v[i] * norm;
+                for (int i = 0; i < 16; i += 2) {
+                    const float y0 = v[i] * norm, y1 = v[i + 1] * norm;
+                    const h2 y = norm == 1.f ? __builtin_convertvector((f2){y0, y1}, h2) : to_half2(y0, y1);
                     // element of the group: c + 16 i (GROUP 256); c + 16 i and c + 8 + 16 (i - 8) (GROUP 128)
-                    dst[GROUP == 256 ? c + 16 * i : c + (i < 8 ? 16 * i : 8 + 16 * (i - 8))] = to_half(y);
-                    mx = fmaxf(mx, fabsf(y));
+                    dst[GROUP == 256 ? c + 16 * i : c + (i < 8 ? 16 * i : 8 + 16 * (i - 8))] = y[0];
+                    dst[GROUP == 256 ? c + 16 * i + 16 : c + (i < 8 ? 16 * i + 16 : 8 + 16 * (i - 7))] = y[1];
+                    mx = fmaxf(fmaxf(mx, fabsf(y0)), fabsf(y1));
                 }
             }
             wave_sync();
         }
     }
-    mx = rows_max(row_max16(mx));  // the wave's maximum (exact in any order)
-    __syncthreads();
+    mx = wave_max(mx);
     if (lane == 0) red[wave] = mx;
     __syncthreads();
     mx = red[0];
@@ -319,7 +346,11 @@ __global__ __launch_bounds__(NW * 64) void rot_quant_kernel(const half_t* __rest
     const float scale = I4 ? fmaxf(mx, 1e-10f) / 7.f : fmaxf(mx / 127.f, 1e-30f);
     if (t == 0) as[row] = scale;
 
-    const float rcp = 1.f / scale;
+    // f / scale as f rcp + f low, rcp + low = 1 / scale to twice the precision: for every fp16 f within the row's maximum that is
+    // the correctly rounded quotient (tests/exhaustive_quotient.c goes through every pair), in two instructions that read
+    // the fp16 value, where div_by_scale takes a conversion and three. The row's scale is infinite only if its maximum is:
+    // every quotient is NaN then, as f / scale corrected by its residual would be.
+    const float rcp = 1.f / scale, low = __builtin_fmaf(-scale, rcp, 1.f) * rcp;
     int8_t* out = Aq + (size_t)row * K;
     // The 16 codes of the row's chunk ch (values 16 ch ..) from its fp16 values lo, hi, stored in one 16-byte write.
     auto quant16 = [&](const h8 lo, const h8 hi, int ch) __attribute__((always_inline)) {
@@ -327,19 +358,13 @@ __global__ __launch_bounds__(NW * 64) void rot_quant_kernel(const half_t* __rest
         int q[16];
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            const float f = (float)(i < 8 ? lo[i] : hi[i - 8]);
-            // f / scale as div_by_scale, its first product f * rcp taken straight from the fp16 value (one mixed-precision
-            // FMA, + 0, in place of a conversion and a multiply: the same value, up to the sign of a zero, which the
-            // code does not depend on).
-            const u32 w = i < 8 ? wl[i >> 1] : wh[(i - 8) >> 1];
-            float y;
-            if (i & 1) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(y) : "v"(w), "v"(rcp));
-            else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(y) : "v"(w), "v"(rcp));
-            const float d = __builtin_fmaf(__builtin_fmaf(-y, scale, f), rcp, y);
+            const u32 w = i < 8 ? wl[i >> 1] : wh[(i - 8) >> 1];  // the value f is its low or high half
+            const float d = i & 1 ? mix<true>(w, rcp, mix<true>(w, low)) : mix<false>(w, rcp, mix<false>(w, low));
             // int8_gemm.hip:84 and :53. The clamp to [lo, hi] (integers) goes before the rounding: both orders give the same
-            // code for every input, NaN included (-128 / -7), and floor then truncation fuse into one conversion.
-            if (I4) q[i] = (int)rintf(fminf(fmaxf(d, -7.f), 7.f));
-            else q[i] = cvt_floor(fminf(fmaxf(d + 0.5f, -128.f), 127.f));
+            // code for every input, NaN included (-128 / -7; the median of a NaN and two numbers is their minimum), and the
+            // + 0.5 and the floor are one conversion (the fp32 sum never rounds past an integer for these quotients: same test).
+            if (I4) q[i] = (int)rintf(__builtin_amdgcn_fmed3f(d, -7.f, 7.f));
+            else q[i] = cvt_nearest_up(__builtin_amdgcn_fmed3f(d, -128.f, 127.f));
         }
         u4v o;
         if constexpr (IL) {

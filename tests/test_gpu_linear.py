@@ -114,6 +114,33 @@ def test_rot_quant_wave_counts_bit_exact(dev, act, M, K, group):
     assert_same(q_of(packed, M, K), q_ref)
 
 
+@pytest.mark.parametrize("kind,K,group", [("int8", 1280, 256), ("int8", 640, 128), ("int4", 1280, 256), ("int4", 640, 128), ("plain", 1040, 0)])
+def test_quantizer_row_ranges_bit_exact(dev, kind, K, group):
+    """Rows of every magnitude fp16 has, from its smallest subnormals (all values within 16 units of 2^-24) to maxima near 4000
+    (rotated values below 65504), multiples of the maximum's 1/254 (quotients that end in one half), and a row of zeros;
+    K leaves the last pass of a wave partly empty."""
+    print(f"row ranges {kind} K={K} group={group}", flush=True)
+    g, k, M = gen(K + group), kern(), 64
+    x = torch.randint(-16, 17, (M, K), generator=g).float() * 2.0**-24
+    for r in range(1, 36):
+        x[r] = torch.randn(K, generator=g) * 2.0 ** (r - 25)
+    for r in range(36, M - 1):
+        x[r] = torch.randint(-254, 255, (K,), generator=g) * 2.0 ** (r - 54)
+    x[M - 1] = 0
+    x = x.clamp(-4000, 4000).half()
+    if kind == "plain":
+        packed, scale = int8_gemm.quantize(k.quant_pack_a, x.to(dev), K)
+        q_ref, s_ref = oracle.quant_rows(x.numpy())
+    elif kind == "int8":
+        packed, scale = int8_gemm.quantize(k.rot_quant_pack_a, x.to(dev), K, group=group)
+        q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), group=group)
+    else:
+        packed, scale = int8_gemm.quantize(k.rot_quant_pack_a_i4, x.to(dev), K, group=group)
+        q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), group=group, i4=True)
+    assert_same(scale.cpu().numpy(), s_ref)
+    assert_same(q_of(packed, M, K), q_ref)
+
+
 @pytest.mark.parametrize("B,L,K", [(1, 77, 3072), (2, 40, 1024)])
 def test_mod_rot_quant_bit_exact(dev, B, L, K):
     print(f"mod_rot_quant B={B} L={L} K={K}", flush=True)
