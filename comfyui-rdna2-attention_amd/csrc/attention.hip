@@ -20,7 +20,9 @@
 // than once per four (copies measured at ~8% of the kernel). A workgroup's rows then lie in one head
 // or two; with two it keeps a second set of tiles, copied by waves 8-11 (waves 0-7 copy the first),
 // and each wave reads the set of its own head. Otherwise a workgroup is four waves over 128 rows of
-// one head, three to a CU. Block ids are remapped so that the workgroups an XCD runs together cover
+// one head, three to a CU; and where such a grid is at most one workgroup per CU, workgroups of 128, 64 or 32 rows whose keys are
+// split between three groups of waves (group j walks tiles j, j + 3, ... with tile stages of its own), which add up their O
+// at the end. Block ids are remapped so that the workgroups an XCD runs together cover
 // a contiguous range of heads and share their K/V through that XCD's L2.
 //
 // Tiles. Each workgroup keeps 32-key tiles of K and V (one or two sets) in three LDS stages. They are copied by
@@ -75,9 +77,16 @@ struct Tile {
     static constexpr int V_BYTES = KB * 256;
     static constexpr int BYTES = K_BYTES + V_BYTES;  // one tile: K, then V
 };
-// Three stages, each of one tile (four waves) or of two, one per head among the workgroup's rows (twelve waves).
-template <bool I8, int NWV>
-constexpr int attn_lds() { return 3 * (NWV == 12 ? 2 : 1) * Tile<I8>::BYTES; }
+// A workgroup: NR waves of 32 query rows, times NS groups of such waves that share the keys out among them.
+#define SPLIT 3                           // key groups of the split layouts
+#define MERGE_BYTES (64 * 64 * 4 + 64 * 8)  // a wave's O, m and l at the end of a split layout
+// Three stages, each of a tile per key group or (twelve waves of rows) one per head among the workgroup's rows; the split layouts'
+// waves past the first group leave their results there at the end, and every wave turns its 32 output rows around there.
+template <bool I8, int NR, int NS>
+constexpr int attn_lds() {
+    const int tiles = 3 * (NR == 12 ? 2 : NS) * Tile<I8>::BYTES, end = NS > 1 ? (NS - 1) * NR * MERGE_BYTES : NR * 32 * 256;
+    return tiles > end ? tiles : end;
+}
 
 typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
 typedef __attribute__((address_space(3))) fp16x4_t lds_fp16x4_t;
@@ -100,23 +109,30 @@ template <int N>
 __device__ __forceinline__ constexpr std::integral_constant<int, (N + 1) % 3> next_stage(std::integral_constant<int, N>) { return {}; }
 __device__ __forceinline__ int next_stage(int s) { return s == 2 ? 0 : s + 1; }
 
-template <bool I8, int NWV>
-__global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_kernel(AttnArgs p) {
+template <bool I8, int NR, int NS>
+__global__ __launch_bounds__(64 * NR * NS) __attribute__((amdgpu_waves_per_eu(NR * NS < 12 && NS > 1 ? 2 : 3, NR * NS < 12 && NS > 1 ? 2 : 3))) void attn_kernel(AttnArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     using T = Tile<I8>;
     // LDS: the K tiles of the three stages, then their V tiles (stage s, set c: K at s KS + c K_BYTES, V at
     // VOFF + s VS + c V_BYTES), so that a stage's offset from the K or V base register fits the 16-bit offset field
     // of an LDS read in every stage (with K and V stages interleaved, the third began at 64 KiB and each of its reads
     // took a v_add).
-    constexpr int NSET = NWV == 12 ? 2 : 1;
+    constexpr bool FLAT = NR == 12;  // the rows flattened over (batch, head, row)
+    static_assert(!FLAT || NS == 1);
+    constexpr int NSET = FLAT ? 2 : NS;
     constexpr int KS = NSET * T::K_BYTES, VS = NSET * T::V_BYTES, VOFF = 3 * KS;
     const int t = threadIdx.x, lane = t & 63, g = lane >> 5, lq = lane & 31;
-    const int wq = __builtin_amdgcn_readfirstlane(t >> 6);  // scalar
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // scalar
+    const int grp = wave / NR, wq = wave % NR;                 // key group, and wave of it
 
     // Block remap: consecutive block ids go round-robin to the 8 XCDs; give each XCD a contiguous run
-    // of (head, q-block) work so its resident workgroups share K/V through its L2.
+    // of (head, q-block) work so its resident workgroups share K/V through its L2 (the first XCDs one more block each
+    // where the grid is no multiple of 8).
     int blk = blockIdx.x;
-    if (p.nblocks % 8 == 0) blk = (blk % 8) * (p.nblocks / 8) + blk / 8;
+    {
+        const int xcd = blk % 8, run = p.nblocks / 8, rest = p.nblocks % 8;
+        blk = xcd * run + min(xcd, rest) + blk / 8;
+    }
     // The wave's query rows q0 .. q0 + 31 of head h of batch b. Tile set c of the workgroup holds the K/V of batch
     // kvb[c], KV head kvh[c]; the wave reads set `set`. Four waves: one set, 128 rows of one head. Twelve waves: 384
     // consecutive rows of the (batch, head, row) range with each head's rows padded to a multiple of 32 (Lq_pad), i.e.
@@ -124,11 +140,12 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
     // rows recompute row Lq - 1 and waves past the last row the last 32 rows, neither stored.
     int b, h, q0, set = 0, kvb[2], kvh[2];
     bool store = true, two = false;
-    if constexpr (NWV == 4) {
+    if constexpr (!FLAT) {
         const int bh = blk / p.qblocks, qblk = blk % p.qblocks;
         b = bh / p.H;
         h = bh % p.H;
-        q0 = qblk * QB + wq * 32;
+        q0 = (qblk * NR + wq) * 32;
+        set = grp;
         kvb[0] = kvb[1] = b;
         kvh[0] = kvh[1] = h / (p.H / p.Hkv);
     } else {
@@ -146,17 +163,119 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
         kvh[1] = (bh1 % p.H) / (p.H / p.Hkv);
     }
 
-    // Q as the B operand of S^T = K Q^T, for the lane's row q0 + lq.
+    // Copy duty: the waves of a key group copy its tiles together; of twelve waves of rows, waves 0-7 copy set 0 and waves 8-11
+    // set 1 (if any).
+    const int cset = FLAT ? (wq >= 8 ? 1 : 0) : grp, cw = FLAT ? wq - 8 * cset : wq;  // the wave's set and index among its copiers
+    const int chead = FLAT ? cset : 0;
+    const bool copier = !FLAT || cset == 0 || two;
+    const half_t* kbase = p.k + kvb[chead] * p.skb + kvh[chead] * p.skh;
+    const half_t* vbase = p.v + kvb[chead] * p.svb + kvh[chead] * p.svh;
+    const int bkv = kvb[chead] * p.Hkv + kvh[chead];
+    const int8_t* k8base = I8 ? p.k8 + (size_t)bkv * p.Lk_pad * 128 : nullptr;
+    const float* ksbase = I8 ? p.ks + (size_t)bkv * p.Lk_pad : nullptr;
+    // Key group grp takes every NS-th tile: its i-th is tile NS i + grp.
+    const int all_tiles = (p.Lk + KB - 1) / KB, tiles = (all_tiles - grp + NS - 1) / NS;
+    auto key_of = [&](int i) __attribute__((always_inline)) { return (NS * i + grp) * KB; };
+
+    // Copies the tile at key0 into stage st, each copying wave its part: a tile is eight DMAs of four K rows and eight of four V rows;
+    // DMA i of copier cw of NC is the (NC i + cw)-th, rows 4 NC i + row0, row0 = 4 cw + lane / 16 (NC = 8 for set 0 of twelve
+    // waves of rows, 4 for its set 1, else the waves of a key group). int8 K: four DMAs of eight rows, rows 8 (NC i + cw) +
+    // lane / 8, and copier 0 the scales. Rows past Lk re-read row Lk - 1: their scores are masked to -1e30, so P is 0 there and
+    // the (finite) values drop out. int8 K is zero-padded to a whole tile by pack_k_i8. Per-lane byte offsets are fixed; only the
+    // tile base moves (the launcher keeps 32 rows of stride inside 2^31 bytes).
+    constexpr int NC = FLAT ? 4 : NR;
+    const bool single = FLAT && cset == 0;  // one K and one V DMA
+    const int row0 = 4 * cw + (lane >> 4);
+    const long skl2 = p.skl * 2, svl2 = p.svl * 2;
+    const int vc = (lane & 15) ^ ((lane >> 4) << 2);
+    // The K chunk's swizzle follows the row: with fewer than four copiers it changes from DMA to DMA (period 4 / NC).
+    u32 k_off[4 / NC];
+#pragma unroll
+    for (int i = 0; i < 4 / NC; i++) k_off[i] = (u32)(row0 * skl2) + ((u32)((lane & 15) ^ ((4 * NC * i + row0) & 15)) << 4);
+    const u32 v_off = (u32)(row0 * svl2) + ((u32)vc << 4);
+    const u32 k8_off = (u32)((8 * cw + (lane >> 3)) * 128) + ((u32)((lane & 7) ^ (lane >> 3)) << 4);
+    auto issue = [&](int key0, int stage) {
+        if (!copier) return;
+        const char* kst = smem + stage * KS + cset * T::K_BYTES;
+        const char* vst = smem + VOFF + stage * VS + cset * T::V_BYTES;
+        if (I8) {
+            if (cw < 4) {
+#pragma unroll
+                for (int i = 0; i < 4 / NC; i++) dma16((const char*)k8base + (size_t)(key0 + 8 * NC * i) * 128, k8_off, kst + (NC * i + cw) * 1024);
+            }
+            if (cw == 0) dma4(ksbase + key0, (u32)min(lane, KB - 1) * 4, kst + KB * 128);
+        }
+        const char* kt = (const char*)kbase + key0 * skl2;
+        const char* vt = (const char*)vbase + key0 * svl2;
+        if (key0 + KB <= p.Lk) {
+            if (single) {
+                if (!I8) dma16(kt, k_off[0], kst + cw * 1024);
+                dma16(vt, v_off, vst + cw * 1024);
+            } else {
+                if (!I8) {
+#pragma unroll
+                    for (int i = 0; i < 8 / NC; i++) dma16(kt + i * 4 * NC * skl2, k_off[i % (4 / NC)], kst + (NC * i + cw) * 1024);
+                }
+#pragma unroll
+                for (int i = 0; i < 8 / NC; i++) dma16(vt + i * 4 * NC * svl2, v_off, vst + (NC * i + cw) * 1024);
+            }
+        } else {
+            // The tile's base stays in SGPRs; the lane's row (clamped to Lk - 1) enters through its 32-bit offset. The
+            // lane id is read again here (a volatile read the compiler cannot hoist), so that this branch, taken once,
+            // holds no registers across the tile loop.
+            u32 ln;
+            asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+            const int r0 = 4 * cw + (int)(ln >> 4);
+            const u32 vcl = ((ln & 15) ^ ((ln >> 4) << 2)) << 4;
+#pragma unroll
+            for (int i = 0; i < 8 / NC; i++) {
+                if (single && i > 0) break;
+                const int ri = single ? r0 : 4 * NC * i + r0, di = single ? cw : NC * i + cw;
+                const u32 r = (u32)(min(key0 + ri, p.Lk - 1) - key0), kcl = ((ln & 15) ^ (u32)(ri & 15)) << 4;
+                if (!I8) dma16(kt, r * (u32)skl2 + kcl, kst + di * 1024);
+                dma16(vt, r * (u32)svl2 + vcl, vst + di * 1024);
+            }
+        }
+    };
+
+    auto first_stage = [](int n) { return ((1 - n) % 3 + 3) % 3; };  // the stage of the first of n tiles (the tile loop)
+    const int first = first_stage(tiles);
+    issue(key_of(0), first);
+    if (tiles > 1) issue(key_of(1), next_stage(first));
+
+    // Q as the B operand of S^T = K Q^T, for the lane's row q0 + lq. The first tiles are on their way by now, so that one memory
+    // latency covers both. Read straight from memory, each load touches 32 rows; in the split layouts, whose key groups need the
+    // same rows, they come once by copies of four rows each, through the LDS stages that the groups' third tiles will fill
+    // (chunk c of row r at c ^ (r & 15); the rows of wave j < 3 of a group where set j's V tile will be, those of wave 3 in two
+    // halves where the K tiles of sets 0 and 1 will be): 2.2 us less at B = 1, H = 24, L = 1101.
     h8 qf[8];
     i4v q8f[4];
     float score_scale = p.scale_log2;
     {
         const int qrow = min(q0 + lq, p.Lq - 1);
-        const half_t* qp = p.q + b * p.sqb + h * p.sqh + (long)qrow * p.sql;
+        const half_t* qhead = p.q + b * p.sqb + h * p.sqh;
+        const half_t* qp = qhead + (long)qrow * p.sql;
+        const char *ql0 = nullptr, *ql1 = nullptr;  // rows 0-15 and 16-31
+        if constexpr (NS > 1) {
+            const int qb = min(q0, p.Lq - 1);
+            auto third = [&](int j) { return next_stage(next_stage(first_stage((all_tiles - j + NS - 1) / NS))); };
+            ql0 = wq < NS ? smem + VOFF + third(wq) * VS + wq * T::V_BYTES : smem + third(0) * KS;
+            ql1 = wq < NS ? ql0 + 4096 : smem + third(1) * KS + T::K_BYTES;
+            for (int i = grp; i < 8; i += NS) {
+                const int r = 4 * i + (lane >> 4);
+                dma16(qhead + (long)qb * p.sql, (u32)(min(q0 + r, p.Lq - 1) - qb) * (u32)(p.sql * 2) + (u32)(((lane & 15) ^ (r & 15)) << 4), (i < 4 ? ql0 : ql1) + (i & 3) * 1024);
+            }
+            wait_copies();
+            __syncthreads();
+        }
+        auto q_chunk = [&](int c) __attribute__((always_inline)) {
+            if constexpr (NS > 1) return *(const h8*)((lq < 16 ? ql0 : ql1) + (lq & 15) * 256 + ((c ^ (lq & 15)) << 4));
+            else return *(const h8*)(qp + c * 8);
+        };
         if (!I8) {
 #pragma unroll
             for (int ks = 0; ks < 8; ks++) {
-                qf[ks] = *(const h8*)(qp + ks * 16 + g * 8);
+                qf[ks] = q_chunk(2 * ks + g);
                 asm volatile("" : "+v"(qf[ks]));  // the loads complete here, not inside the tile loop
             }
         } else {
@@ -164,8 +283,8 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
             float qmax = 0.f;
 #pragma unroll
             for (int ks = 0; ks < 4; ks++) {
-                raw[2 * ks] = *(const h8*)(qp + ks * 32 + g * 16);
-                raw[2 * ks + 1] = *(const h8*)(qp + ks * 32 + g * 16 + 8);
+                raw[2 * ks] = q_chunk(4 * ks + 2 * g);
+                raw[2 * ks + 1] = q_chunk(4 * ks + 2 * g + 1);
             }
 #pragma unroll
             for (int i = 0; i < 8; i++)
@@ -175,95 +294,31 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
             qmax = fmaxf(qh[0], qh[1]);
             const float q_scale = fmaxf(qmax / 127.f, 1e-30f);  // hip_attention.hip:183
             score_scale = q_scale * p.scale_log2;
-            const float q_rcp = 1.f / q_scale;
+            // q / q_scale from a two-term reciprocal (correctly rounded, as in quant.hip), and its rounding by adding 3 x 2^22, whose low
+            // byte is then the code (hip_attention.hip:192; a NaN's is 0): 3.75 instructions per value where a conversion, div_by_scale,
+            // rintf, a mask and a shift took eight, three times over in the split layouts.
+            const float q_rcp = 1.f / q_scale, q_low = __builtin_fmaf(-q_scale, q_rcp, 1.f) * q_rcp;
 #pragma unroll
             for (int ks = 0; ks < 4; ks++) {
                 u4v w;
 #pragma unroll
                 for (int d = 0; d < 4; d++) {
-                    u32 x = 0;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const int idx = d * 4 + e;
-                        const float f = (float)raw[2 * ks + (idx >> 3)][idx & 7];
-                        x |= (u32)((int)rintf(div_by_scale(f, q_scale, q_rcp)) & 255) << (e * 8);  // f / q_scale, hip_attention.hip:192
-                    }
-                    w[d] = x;
+                    const u4v words = __builtin_bit_cast(u4v, raw[2 * ks + (d >> 1)]);
+                    const u32 w0 = words[2 * (d & 1)], w1 = words[2 * (d & 1) + 1];
+                    auto code = [&](float f) { return (int)__float_as_uint(f + 12582912.f); };
+                    w[d] = pack4(code(mix<false>(w0, q_rcp, mix<false>(w0, q_low))), code(mix<true>(w0, q_rcp, mix<true>(w0, q_low))),
+                                 code(mix<false>(w1, q_rcp, mix<false>(w1, q_low))), code(mix<true>(w1, q_rcp, mix<true>(w1, q_low))));
                 }
                 q8f[ks] = as_i4(w);
             }
         }
+        if constexpr (NS > 1) __syncthreads();  // every wave has its Q
     }
 
     f16v o[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) o[i] = (f16v){};
     float m = -1e30f, l = 0.f;
-
-    // Copy duty: four waves copy the tile together; of twelve, waves 0-7 copy set 0 and waves 8-11 set 1 (if any).
-    const int cset = NWV == 12 && wq >= 8 ? 1 : 0, cw = wq - 8 * cset;  // the wave's set and index among its copiers
-    const bool copier = cset == 0 || two;
-    const half_t* kbase = p.k + kvb[cset] * p.skb + kvh[cset] * p.skh;
-    const half_t* vbase = p.v + kvb[cset] * p.svb + kvh[cset] * p.svh;
-    const int bkv = kvb[cset] * p.Hkv + kvh[cset];
-    const int8_t* k8base = I8 ? p.k8 + (size_t)bkv * p.Lk_pad * 128 : nullptr;
-    const float* ksbase = I8 ? p.ks + (size_t)bkv * p.Lk_pad : nullptr;
-    const int tiles = (p.Lk + KB - 1) / KB;
-
-    // Copies the tile at key0 into stage st, each copying wave its part: DMA i (< 2) of a wave fills K (and V)
-    // rows 16 i + row0 .. +3, row0 = 4 cw + lane / 16; the eight copiers of set 0 among twelve waves take one DMA
-    // each, rows row0 .. + 3 (int8 K: one DMA for each of copiers 0-3, rows 8 cw + lane / 8, and copier 0 the
-    // scales). Rows past Lk re-read row Lk - 1: their scores are masked to -1e30, so P is 0 there and the (finite)
-    // values drop out. int8 K is zero-padded to a whole tile by pack_k_i8. Per-lane byte offsets are fixed; only the
-    // tile base moves (the launcher keeps 32 rows of stride inside 2^31 bytes).
-    constexpr bool ONE = NWV == 12;  // one K and one V DMA for the copiers of set 0 (two otherwise)
-    const bool single = ONE && cset == 0;
-    const int row0 = 4 * cw + (lane >> 4);
-    const long skl2 = p.skl * 2, svl2 = p.svl * 2;
-    const int kc = (lane & 15) ^ (row0 & 15), vc = (lane & 15) ^ ((lane >> 4) << 2);
-    const u32 k_off = (u32)(row0 * skl2) + ((u32)kc << 4);
-    const u32 v_off = (u32)(row0 * svl2) + ((u32)vc << 4);
-    const u32 k8_off = (u32)((8 * cw + (lane >> 3)) * 128) + ((u32)((lane & 7) ^ (lane >> 3)) << 4);
-    auto issue = [&](int key0, int stage) {
-        if (!copier) return;
-        const char* kst = smem + stage * KS + cset * T::K_BYTES;
-        const char* vst = smem + VOFF + stage * VS + cset * T::V_BYTES;
-        if (I8) {
-            if (cw < 4) dma16((const char*)k8base + (size_t)key0 * 128, k8_off, kst + cw * 1024);
-            if (cw == 0) dma4(ksbase + key0, (u32)min(lane, KB - 1) * 4, kst + KB * 128);
-        }
-        const char* kt = (const char*)kbase + key0 * skl2;
-        const char* vt = (const char*)vbase + key0 * svl2;
-        if (key0 + KB <= p.Lk) {
-            if (single) {
-                if (!I8) dma16(kt, k_off, kst + cw * 1024);
-                dma16(vt, v_off, vst + cw * 1024);
-            } else {
-                if (!I8) {
-#pragma unroll
-                    for (int i = 0; i < 2; i++) dma16(kt + i * 16 * skl2, k_off, kst + (4 * i + cw) * 1024);
-                }
-#pragma unroll
-                for (int i = 0; i < 2; i++) dma16(vt + i * 16 * svl2, v_off, vst + (4 * i + cw) * 1024);
-            }
-        } else {
-            // The tile's base stays in SGPRs; the lane's row (clamped to Lk - 1) enters through its 32-bit offset. The
-            // lane id is read again here (a volatile read the compiler cannot hoist), so that this branch, taken once,
-            // holds no registers across the tile loop.
-            u32 ln;
-            asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-            const int r0 = 4 * cw + (int)(ln >> 4);
-            const u32 kcl = ((ln & 15) ^ (u32)(r0 & 15)) << 4, vcl = ((ln & 15) ^ ((ln >> 4) << 2)) << 4;
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                if (single && i > 0) break;
-                const int ri = single ? r0 : 16 * i + r0, di = single ? cw : 4 * i + cw;
-                const u32 r = (u32)(min(key0 + ri, p.Lk - 1) - key0);
-                if (!I8) dma16(kt, r * (u32)skl2 + kcl, kst + di * 1024);
-                dma16(vt, r * (u32)svl2 + vcl, vst + di * 1024);
-            }
-        }
-    };
 
     // LDS offsets of the lane's V^T reads (and int8 K reads) within a stage, fixed for the whole loop: the stage
     // enters as an immediate offset (the loop below is unrolled over the two stages), so the tile loop spends
@@ -397,6 +452,22 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
         }
     };
     auto exps = [&](int k) __attribute__((always_inline)) { exps_into(s, k, pf[0], pf[1]); };
+    // The rule of the lazy rescale for the scores in s: their maximum over the row, and m + 8. (The maximum reads the products'
+    // results through compiler-visible operations: the compiler inserts the wait states a VALU read of an MFMA result needs
+    // only for instructions it can see, not inline asm.)
+    auto row_max = [&]() __attribute__((always_inline)) {
+        float mx = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[r]);
+        const f2 mh = halves(mx);
+        return fmaxf(mh[0], mh[1]) * (I8 ? score_scale : p.scale_log2);
+    };
+    // The first tile always moves m (from -1e30; O and l are zero): done before its exponentials are made, which spares
+    // making them twice (settle below): 0.3-1.1 us of a call.
+    auto first_max = [&]() __attribute__((always_inline)) {
+        const float mx = row_max();
+        if (__any(mx > m + 8.f)) m = fmaxf(m, mx);
+    };
     // fp16: part k (< 4: keys 0-15) of the next tile's P into registers of its own, pinned where it is issued (the
     // empty asm consumes the results: without it the parts placed beside the PV products sink past the step's
     // closing barrier to their first use).
@@ -407,21 +478,13 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
     // The lazy rescale (hip_attention.hip:333-340): m moves only when some row's tile maximum exceeds m + 8. The tile's P
     // is first made with the current m; a row whose maximum exceeds m + 8 has a P of at least ~2^7.8 in one of its two
     // lanes, so a lane sum that grew by no more than 64 (and is not NaN) proves that no row needs the rescale, and the
-    // P just made is the one the rule gives. Otherwise (always on the first tile, where m is -1e30 and P overflows,
-    // rarely after) the scores are recomputed from the tile still in LDS, the rule is applied to their maxima, and P
+    // P just made is the one the rule gives. Otherwise (rarely after the first tile) the scores are recomputed from the tile still in LDS, the rule is applied to their maxima, and P
     // and l are made again from the old l -- the same values, in the same order, as applying the rule first.
     auto settle = [&](auto stage, int key0, auto last, float l_old) __attribute__((always_inline)) {
         if (__builtin_expect(__any(!(l <= l_old + 64.f)), 0)) {
             qk(stage, s, no_hook);
             if constexpr (decltype(last)::value) mask(s, key0);
-            // The maximum reads the products' results through compiler-visible operations: the compiler inserts
-            // the wait states a VALU read of an MFMA result needs only for instructions it can see, not inline asm.
-            float mx = s[0];
-#pragma unroll
-            for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[r]);
-            const f2 mh = halves(mx);
-            mx = fmaxf(mh[0], mh[1]);
-            mx *= I8 ? score_scale : p.scale_log2;
+            const float mx = row_max();
             l = l_old;
             if (__any(mx > m + 8.f)) {
                 const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - mn);
@@ -490,20 +553,20 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
     auto step = [&](int i, auto stage, auto kind) __attribute__((always_inline)) {
         constexpr int K = decltype(kind)::value;
         const auto next = next_stage(stage);
-        if constexpr (K == 0) issue((i + 2) * KB, (int)next_stage(next));
+        if constexpr (K == 0) issue(key_of(i + 2), (int)next_stage(next));
         if constexpr (I8) l_old = l;
         if constexpr (K != 2) {
             float nxt[16];
             if constexpr (I8) {
                 i16v raw;
                 qk_raw(next, raw, exps);
-                settle(stage, i * KB, std::false_type{}, l_old);
+                settle(stage, key_of(i), std::false_type{}, l_old);
                 pv(stage, [&](int dt) { scale_part(next, raw, nxt, dt); }, no_hook);
-                if constexpr (K == 1) mask(nxt, (i + 1) * KB);
+                if constexpr (K == 1) mask(nxt, key_of(i + 1));
             } else {
                 qk(next, nxt, [&](int k) { if (k & 1) exps(4 + (k >> 1)); });
-                if constexpr (K == 1) mask(nxt, (i + 1) * KB);
-                settle(stage, i * KB, std::false_type{}, l_old);
+                if constexpr (K == 1) mask(nxt, key_of(i + 1));
+                settle(stage, key_of(i), std::false_type{}, l_old);
                 l_old = l;
                 h8 pn;
                 pv(stage, [&](int dt) { if (dt & 1) exps_to(nxt, dt >> 1, pn); }, [&](int dt) { if (dt & 1) exps_to(nxt, 2 + (dt >> 1), pn); });
@@ -514,7 +577,7 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
         } else {
 #pragma unroll
             for (int k = I8 ? 0 : PARTS / 2; k < PARTS; k++) exps(k);
-            settle(stage, i * KB, std::true_type{}, l_old);
+            settle(stage, key_of(i), std::true_type{}, l_old);
             pv(stage, no_hook, no_hook);
         }
         if constexpr (K == 0) {
@@ -522,20 +585,21 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
             __syncthreads();
         }
     };
-    const int first = ((1 - tiles) % 3 + 3) % 3;  // the stage of tile 0
-    issue(0, first);
-    if (tiles > 1) issue(KB, next_stage(first));
-    wait_copies();
-    __syncthreads();
+    if constexpr (NS == 1) {  // split: already waited for, with Q
+        wait_copies();
+        __syncthreads();
+    }
     if (tiles == 1) {
         qk(S0{}, s, no_hook);
-        mask(s, 0);
+        mask(s, key_of(0));
+        first_max();
         if constexpr (!I8)
 #pragma unroll
             for (int k = 0; k < PARTS / 2; k++) exps(k);
         step(0, S0{}, Last{});
     } else {
         qk(first, s, no_hook);
+        first_max();
         if constexpr (!I8)
 #pragma unroll
             for (int k = 0; k < PARTS / 2; k++) exps(k);
@@ -557,11 +621,60 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
         step(tiles - 1, S0{}, Last{});
     }
 
+    // Key groups: those past the first leave O, m and l in LDS (in the order of their registers, 16 bytes per lane), and the first
+    // adds them to its own, all scaled to the largest of the groups' maxima. A group with a tile fewer than the first has met a
+    // barrier fewer.
+    if constexpr (NS > 1) {
+        const int most = (all_tiles + NS - 1) / NS;
+        if (max(tiles - 2, 0) < max(most - 2, 0)) __syncthreads();
+        __syncthreads();  // the tiles have been read
+        if (grp > 0) {
+            char* to = smem + ((grp - 1) * NR + wq) * MERGE_BYTES;
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+                for (int r4 = 0; r4 < 4; r4++)
+                    *(f4*)(to + (dt * 4 + r4) * 1024 + lane * 16) = (f4){o[dt][r4 * 4], o[dt][r4 * 4 + 1], o[dt][r4 * 4 + 2], o[dt][r4 * 4 + 3]};
+            *(f2*)(to + 16384 + lane * 8) = (f2){m, l};
+        }
+        __syncthreads();
+        if (grp > 0) return;
+        f2 ml[NS - 1];
+        float top = m;
+#pragma unroll
+        for (int j = 0; j < NS - 1; j++) {
+            ml[j] = *(const f2*)(smem + (j * NR + wq) * MERGE_BYTES + 16384 + lane * 8);
+            top = fmaxf(top, ml[j][0]);
+        }
+        const float own = __builtin_amdgcn_exp2f(m - top);
+        l *= own;
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) o[dt] *= own;
+#pragma unroll
+        for (int j = 0; j < NS - 1; j++) {
+            const float a = __builtin_amdgcn_exp2f(ml[j][0] - top);
+            l = __builtin_fmaf(ml[j][1], a, l);
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++) {
+#pragma unroll
+                for (int r4 = 0; r4 < 4; r4++) {
+                    const f4 x = *(const f4*)(smem + (j * NR + wq) * MERGE_BYTES + (dt * 4 + r4) * 1024 + lane * 16);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[dt][r4 * 4 + e] = __builtin_fmaf(x[e], a, o[dt][r4 * 4 + e]);
+                }
+                asm volatile("" : "+v"(o[dt]));  // added here, 16 registers of a group at a time
+            }
+        }
+    }
+
     // Normalise and store: the lane halves hold disjoint keys of one row.
     const f2 lh = halves(l);
     const float inv = 1.f / (lh[0] + lh[1]);
-    const int row = q0 + lq;
-    half_t* op = p.o + b * p.sob + h * p.soh + (long)row * p.sol;
+    // The rows turn around in LDS (32 x 256 bytes per wave, 16-byte chunk c of row r at c ^ (r & 15)), so that a store covers four
+    // whole rows: as 8-byte pieces of 32 rows each, the stores took 2.4 us of a four-wave workgroup's time and 4.3 of a
+    // twelve-wave one's.
+    if constexpr (NS == 1) __syncthreads();  // the tiles have been read
+    char* turn = smem + wq * (NS > 1 ? MERGE_BYTES : 32 * 256);  // split: the wave's own part of what it has merged
 #pragma unroll
     for (int dt = 0; dt < 4; dt++)
 #pragma unroll
@@ -569,8 +682,18 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3, 3))
             h4v w;
 #pragma unroll
             for (int e = 0; e < 4; e++) w[e] = to_half(o[dt][r4 * 4 + e] * inv);
-            if (store && row < p.Lq) *(h4v*)(op + dt * 32 + 8 * r4 + 4 * g) = w;
+            *(h4v*)(turn + lq * 256 + (((dt * 4 + r4) ^ (lq & 15)) << 4) + g * 8) = w;
         }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    half_t* op = p.o + b * p.sob + h * p.soh + (lane & 15) * 8;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int r = 4 * i + (lane >> 4), row = q0 + r;
+        const h8 x = *(const h8*)(turn + r * 256 + (((lane & 15) ^ (r & 15)) << 4));
+        if (store && row < p.Lq) *(h8*)(op + (long)row * p.sol) = x;
+    }
 }
 
 // Per-key absmax int8 quantization of K (pack_kv_i8, hip_attention.hip:56-94): 16 lanes per key,
@@ -620,8 +743,7 @@ static AttnArgs make_args(const void* q, const void* k, const void* v, void* out
     a.Lq = Lq;
     a.Lk = Lk;
     a.Lk_pad = (Lk + KB - 1) / KB * KB;
-    a.qblocks = (Lq + QB - 1) / QB;
-    a.nblocks = a.qblocks * B * H;
+    a.qblocks = a.nblocks = 0;  // launch_attn_layout
     a.Lq_pad = (Lq + 31) / 32 * 32;
     a.rows = (long)B * H * a.Lq_pad;
     a.sqb = st[0]; a.sqh = st[1]; a.sql = st[2];
@@ -632,12 +754,17 @@ static AttnArgs make_args(const void* q, const void* k, const void* v, void* out
     return a;
 }
 
-template <bool I8, int NWV>
-static int launch_attn_waves(const AttnArgs& a, void* stream) {
-    constexpr size_t lds = attn_lds<I8, NWV>();
+template <bool I8, int NR, int NS>
+static int launch_attn_layout(AttnArgs a, void* stream) {
+    constexpr size_t lds = attn_lds<I8, NR, NS>();
     static std::atomic<size_t> configured[RDA_MAX_DEVICES];
-    if (const int e = ensure_dynamic_lds((const void*)attn_kernel<I8, NWV>, lds, configured)) return e;
-    hipLaunchKernelGGL((attn_kernel<I8, NWV>), dim3(a.nblocks), dim3(64 * NWV), lds, (hipStream_t)stream, a);
+    if (const int e = ensure_dynamic_lds((const void*)attn_kernel<I8, NR, NS>, lds, configured)) return e;
+    const long bh = a.rows / a.Lq_pad;  // B H
+    a.qblocks = (a.Lq + 32 * NR - 1) / (32 * NR);
+    const long blocks = NR == 12 ? (a.rows + FLAT_ROWS - 1) / FLAT_ROWS : bh * a.qblocks;
+    if (blocks >= 1L << 31) return RDA_ERR_INVALID;
+    a.nblocks = (int)blocks;
+    hipLaunchKernelGGL((attn_kernel<I8, NR, NS>), dim3(a.nblocks), dim3(64 * NR * NS), lds, (hipStream_t)stream, a);
     return (int)hipGetLastError();
 }
 
@@ -656,33 +783,52 @@ static int device_cus(int* cus) {
     return 0;
 }
 
-// Workgroup layout: twelve waves over 384 rows of the (batch, head, row) range (every head of at least 384 query rows,
+// Row strides of K and V must keep a tile's 32 rows within 2^31 bytes (the kernel's 32-bit per-lane offsets).
+// K and V reach LDS by 16-byte global->LDS copies: their base addresses and their (batch, head, row) strides must
+// keep every row 16-byte aligned.
+static bool dma_ready(const void* p, long sb, long sh, long sl) { return ((uintptr_t)p & 15) == 0 && sb % 8 == 0 && sh % 8 == 0 && sl % 8 == 0; }
+
+// Workgroup layout. Unsplit: twelve waves over 384 rows of the (batch, head, row) range (every head of at least 384 query rows,
 // so that a workgroup's rows span at most two heads), or four waves over 128 rows of one head. The twelve-wave grid
 // has a third as many workgroups, one per CU: it is the faster one only when it still covers most of the chip. B = 1,
 // H = 24, fp16, one process: 1024 rows per head (64 twelve-wave workgroups) 45.2 us twelve-wave against 24.6 us
 // four-wave, 2048 (128) 77.7 / 62.4, 2560 (160) 96.0 / 84.5, 2816 (176) 108.6 / 120.1, 3072 (192) 121.1 / 134.7,
 // 4096 (256) 193.0 / 199.6; int8-QK alike, and the outputs bit-identical. So twelve waves when their grid covers at
-// least two thirds of the CUs. waves: 0 chooses so; 4 or 12 fixes the layout (12 needs Lq >= 384).
+// least two thirds of the CUs.
+// Split keys, where 128-row workgroups leave CUs idle or give each SIMD one wave, which then waits out every latency of its
+// tile step alone (0.45 us a tile; three waves of a SIMD take 0.95 us for three): the fewest rows per workgroup whose grid is
+// still one per CU. B = 1, us unsplit / three groups of four, two and one waves: 24 x 1101 fp16 25.8 / 23.4, 31.1, 54.6, int8-QK
+// 24.9 / 23.9, 32.9, 52.0; 8 x 2000 (64-row grid: 256) 37.1 / 30.2, 26.5, 41.5; 2 x 9000 151 / 110, 181, 232; 4 x 1000 by 1152
+// keys 24.6 / 22.3, 17.6, 15.1. A split layout starts and ends ~1 us later than it would unsplit (more to copy first, O added up
+// at the end): 24 x 700 (22 tiles) breaks even, int8-QK at 27 (18.2 / 17.7 at 22, 23.9 / 24.9 at 35). Its sums are
+// those of another order, so the smallest calls, which must keep the bits that both unsplit layouts give (tests/test_gpu_attention.py),
+// stay with those: up to 736 keys, or 128-row workgroups for less than an eighth of the CUs.
+// waves: 0 chooses so; 4 or 12 fixes an unsplit layout (12 needs Lq >= 384); -3, -6 or -12 (that many waves, in three key
+// groups) a split one (more than 64 keys, Q's rows 16-byte aligned).
 template <bool I8>
 static int launch_attn(AttnArgs a, int waves, void* stream) {
     const long flat = (a.rows + FLAT_ROWS - 1) / FLAT_ROWS;
+    // The split layouts need a tile for every key group, and copy Q's rows as K's and V's.
+    const bool split = a.Lk > (SPLIT - 1) * KB && dma_ready(a.q, a.sqb, a.sqh, a.sql) && a.sql >= 0 && a.sql < (1L << 24);
     if (waves == 0) {
         int cus = 0;
         if (const int e = device_cus(&cus)) return e;
-        waves = a.Lq >= FLAT_ROWS && 3 * flat >= 2L * cus ? 12 : 4;
+        const long heads = a.rows / a.Lq_pad;
+        auto grid = [&](int rows) { return heads * ((a.Lq + rows - 1) / rows); };
+        const bool few = split && a.Lk > 23 * KB && 8 * grid(QB) >= cus;
+        if (few && grid(32) <= cus) waves = -3;
+        else if (few && grid(64) <= cus) waves = -6;
+        else if (few && grid(QB) <= cus && (!I8 || a.Lk > 27 * KB)) waves = -12;
+        else waves = a.Lq >= FLAT_ROWS && 3 * flat >= 2L * cus ? 12 : 4;
     }
-    if (waves == 12 && a.Lq >= FLAT_ROWS && flat < (1L << 31)) {
-        a.nblocks = (int)flat;
-        return launch_attn_waves<I8, 12>(a, stream);
-    }
-    if (waves == 4) return launch_attn_waves<I8, 4>(a, stream);
+    if (waves == 12 && a.Lq >= FLAT_ROWS) return launch_attn_layout<I8, 12, 1>(a, stream);
+    if (waves == 4) return launch_attn_layout<I8, 4, 1>(a, stream);
+    if (waves == -12 && split) return launch_attn_layout<I8, 4, SPLIT>(a, stream);
+    if (waves == -6 && split) return launch_attn_layout<I8, 2, SPLIT>(a, stream);
+    if (waves == -3 && split) return launch_attn_layout<I8, 1, SPLIT>(a, stream);
     return RDA_ERR_INVALID;
 }
 
-// Row strides of K and V must keep a tile's 32 rows within 2^31 bytes (the kernel's 32-bit per-lane offsets).
-// K and V reach LDS by 16-byte global->LDS copies: their base addresses and their (batch, head, row) strides must
-// keep every row 16-byte aligned.
-static bool dma_ready(const void* p, long sb, long sh, long sl) { return ((uintptr_t)p & 15) == 0 && sb % 8 == 0 && sh % 8 == 0 && sl % 8 == 0; }
 
 static bool attn_shapes_ok(int B, int H, int Hkv, int Lq, int Lk, const long* st) {
     const bool rows_ok = st[5] >= 0 && st[5] < (1L << 24) && st[8] >= 0 && st[8] < (1L << 24);

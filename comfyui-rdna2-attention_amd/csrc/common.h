@@ -109,6 +109,16 @@ __device__ __forceinline__ float div_by_scale(float x, float s, float rcp) {
     return __builtin_fmaf(__builtin_fmaf(-y, s, x), rcp, y);
 }
 
+// a * s + c in fp32 for the low (HI false) or high fp16 value a of a word: the compiler makes it one mixed-precision FMA
+// (v_fma_mix_f32), without a conversion. With c = 0 it is the fp32 product, up to the sign of a zero, which no code depends on.
+template <bool HI>
+__device__ __forceinline__ float mix(u32 w, float s, float c = 0.f) { return __builtin_fmaf((float)__builtin_bit_cast(h2, w)[HI], s, c); }
+// The low bytes of a, b, c, d as one word (a in the lowest byte): three byte permutes.
+__device__ __forceinline__ u32 pack4(int a, int b, int c, int d) {
+    const u32 ab = __builtin_amdgcn_perm((u32)b, (u32)a, 0x0c0c0400u), cd = __builtin_amdgcn_perm((u32)d, (u32)c, 0x0c0c0400u);
+    return __builtin_amdgcn_perm(cd, ab, 0x05040100u);
+}
+
 __device__ __forceinline__ i4v as_i4(u4v v) { return __builtin_bit_cast(i4v, v); }
 
 // Cross-lane reductions on DPP and lane-swap instructions (one VALU op per step, no LDS round trip).

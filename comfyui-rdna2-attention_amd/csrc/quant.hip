@@ -59,10 +59,6 @@ __device__ __forceinline__ h2 to_half2(float a, float b) {
     asm("" : "+v"(a), "+v"(b));  // round to fp32 first, as in to_half
     return __builtin_convertvector((f2){a, b}, h2);
 }
-// a * s + c in fp32 for the low (HI false) or high fp16 value a of a word: the compiler makes it one mixed-precision FMA
-// (v_fma_mix_f32), without a conversion. With c = 0 it is the fp32 product, up to the sign of a zero, which no code depends on.
-template <bool HI>
-__device__ __forceinline__ float mix(u32 w, float s, float c = 0.f) { return __builtin_fmaf((float)__builtin_bit_cast(h2, w)[HI], s, c); }
 // SwiGLU (int8_gemm.hip:130-132): r16(r16(silu(g)) u) with silu(g) = g / (1 + rda_expf(-g)) in fp32; the sigmoid
 // gate (int8_gemm.hip:135-137): r16(x r16(sigmoid(gate))), sigmoid(g) = 1 / (1 + rda_expf(-g)) in fp32.
 // Both take a fast path -- hardware exp2 of a rounded argument and a hardware reciprocal -- whose value q lies
@@ -125,12 +121,6 @@ __device__ __forceinline__ int cvt_nearest_up(float x) {
     int r;
     asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
     return r;
-}
-
-// The low bytes of a, b, c, d as one word (a in the lowest byte): three byte permutes.
-__device__ __forceinline__ u32 pack4(int a, int b, int c, int d) {
-    const u32 ab = __builtin_amdgcn_perm((u32)b, (u32)a, 0x0c0c0400u), cd = __builtin_amdgcn_perm((u32)d, (u32)c, 0x0c0c0400u);
-    return __builtin_amdgcn_perm(cd, ab, 0x05040100u);
 }
 
 // GROUP 256 or 128 rotates; GROUP 0 is quant_pack_a (no rotation, int8_gemm.hip:93-103). NW waves per row: the

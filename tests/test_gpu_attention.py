@@ -93,6 +93,37 @@ def attention_layout(q, k, v, scale, int8_qk, waves):
     return out
 
 
+# Tiles per key group: 3 tiles (one each), 4 and 5 (the later groups one fewer), 7 and 8 (the same, past the two-tile start),
+# a partial last tile in each group; rows that end inside a wave and leave waves without any; GQA and batch 2.
+@pytest.mark.parametrize("int8_qk", [False, True])
+@pytest.mark.parametrize("B,H,Hkv,Lq,Lk", [(1, 2, 1, 64, 65), (1, 3, 3, 33, 97), (2, 4, 2, 130, 160), (1, 2, 2, 100, 224), (1, 1, 1, 1, 250), (2, 2, 1, 257, 1101)])
+def test_attention_split_keys(dev, int8_qk, B, H, Hkv, Lq, Lk):
+    """Each split layout against the float64 closed form, and bit for bit equal to the others."""
+    print(f"split keys B={B} H={H} Hkv={Hkv} Lq={Lq} Lk={Lk} int8_qk={int8_qk}", flush=True)
+    q, k, v = qkv(B, H, Hkv, Lq, Lk, seed=Lk)
+    ref = (oracle.attention_i8qk_f64 if int8_qk else oracle.attention_f64)(q.numpy(), k.numpy(), v.numpy(), 128 ** -0.5)
+    outs = [attention_layout(q.to(dev), k.to(dev), v.to(dev), 128 ** -0.5, int8_qk, waves) for waves in (-12, -6, -3)]
+    close(outs[0], ref)
+    for out in outs[1:]:
+        assert torch.equal(out.view(torch.int16), outs[0].view(torch.int16))
+
+
+@pytest.mark.parametrize("int8_qk", [False, True])
+@pytest.mark.parametrize("B,H,Lq,Lk", [(1, 8, 400, 736), (2, 4, 400, 737), (1, 31, 100, 740), (1, 8, 2048, 740), (1, 9, 2048, 770), (1, 24, 1281, 900)])
+def test_attention_choice_of_layout(dev, int8_qk, B, H, Lq, Lk):
+    """Either side of each line of the automatic choice, query rows and output being views with odd strides (query rows that
+    are not 16-byte aligned keep an unsplit layout), against the float64 closed form on a sample of rows."""
+    print(f"choice of layout B={B} H={H} Lq={Lq} Lk={Lk} int8_qk={int8_qk}", flush=True)
+    q, k, v = qkv(B, H, H, Lq, Lk, seed=Lq + Lk)
+    rows = torch.cat([torch.arange(0, 40), torch.arange(Lq - 40, Lq)])
+    ref = (oracle.attention_i8qk_f64 if int8_qk else oracle.attention_f64)(q[:, :, rows].numpy(), k.numpy(), v.numpy(), 128 ** -0.5)
+    for pad in (0, 4):
+        views = [torch.zeros(B, Lq, H, 128 + pad, dtype=torch.float16, device=dev)[..., pad:].transpose(1, 2) for _ in range(2)]
+        views[0].copy_(q)
+        hip_attention.attention(views[0], k.to(dev), v.to(dev), views[1], 128 ** -0.5, int8_qk)
+        close(views[1][:, :, rows.to(dev)], ref)
+
+
 @pytest.mark.parametrize("int8_qk", [False, True])
 def test_attention_zero_query_rows(dev, int8_qk):
     """All-zero query rows (the int8 row scale then sits at its 1e-30 floor) with a partial last key tile: the keys past
