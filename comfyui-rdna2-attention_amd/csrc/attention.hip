@@ -64,7 +64,8 @@ struct AttnArgs {
     const float* ks;   // per-key scales [B * Hkv][Lk_pad]
     int H, Hkv, Lq, Lk, Lk_pad, qblocks, nblocks;
     int Lq_pad;  // Lq rounded up to 32: the rows of a head in the flattened range
-    long rows;   // B H Lq_pad, the query rows flattened over (batch, head, row)
+    int head0;   // this launch's first of the B H heads
+    long rows;   // its heads' query rows flattened over (batch, head, row): heads times Lq_pad
     long sqb, sqh, sql, skb, skh, skl, svb, svh, svl, sob, soh, sol;
     float scale_log2;
 };
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(64 * NR * NS) __attribute__((amdgpu_waves_per_eu(NR
     int b, h, q0, set = 0, kvb[2], kvh[2];
     bool store = true, two = false;
     if constexpr (!FLAT) {
-        const int bh = blk / p.qblocks, qblk = blk % p.qblocks;
+        const int bh = p.head0 + blk / p.qblocks, qblk = blk % p.qblocks;
         b = bh / p.H;
         h = bh % p.H;
         q0 = (qblk * NR + wq) * 32;
@@ -151,7 +152,8 @@ __global__ __launch_bounds__(64 * NR * NS) __attribute__((amdgpu_waves_per_eu(NR
     } else {
         const long g0 = (long)blk * FLAT_ROWS, gw = g0 + 32 * wq, gc = gw < p.rows ? gw : p.rows - 32;
         store = gw < p.rows;
-        const int bh = (int)(gc / p.Lq_pad), bh0 = (int)(g0 / p.Lq_pad), bh1 = (int)((min(g0 + FLAT_ROWS, p.rows) - 1) / p.Lq_pad);
+        const int bh = p.head0 + (int)(gc / p.Lq_pad), bh0 = p.head0 + (int)(g0 / p.Lq_pad);
+        const int bh1 = p.head0 + (int)((min(g0 + FLAT_ROWS, p.rows) - 1) / p.Lq_pad);
         b = bh / p.H;
         h = bh % p.H;
         q0 = (int)(gc % p.Lq_pad);
@@ -745,6 +747,7 @@ static AttnArgs make_args(const void* q, const void* k, const void* v, void* out
     a.Lk_pad = (Lk + KB - 1) / KB * KB;
     a.qblocks = a.nblocks = 0;  // launch_attn_layout
     a.Lq_pad = (Lq + 31) / 32 * 32;
+    a.head0 = 0;
     a.rows = (long)B * H * a.Lq_pad;
     a.sqb = st[0]; a.sqh = st[1]; a.sql = st[2];
     a.skb = st[3]; a.skh = st[4]; a.skl = st[5];
@@ -759,9 +762,9 @@ static int launch_attn_layout(AttnArgs a, void* stream) {
     constexpr size_t lds = attn_lds<I8, NR, NS>();
     static std::atomic<size_t> configured[RDA_MAX_DEVICES];
     if (const int e = ensure_dynamic_lds((const void*)attn_kernel<I8, NR, NS>, lds, configured)) return e;
-    const long bh = a.rows / a.Lq_pad;  // B H
+    const long heads = a.rows / a.Lq_pad;
     a.qblocks = (a.Lq + 32 * NR - 1) / (32 * NR);
-    const long blocks = NR == 12 ? (a.rows + FLAT_ROWS - 1) / FLAT_ROWS : bh * a.qblocks;
+    const long blocks = NR == 12 ? (a.rows + FLAT_ROWS - 1) / FLAT_ROWS : heads * a.qblocks;
     if (blocks >= 1L << 31) return RDA_ERR_INVALID;
     a.nblocks = (int)blocks;
     hipLaunchKernelGGL((attn_kernel<I8, NR, NS>), dim3(a.nblocks), dim3(64 * NR * NS), lds, (hipStream_t)stream, a);
@@ -805,30 +808,54 @@ static bool dma_ready(const void* p, long sb, long sh, long sl) { return ((uintp
 // stay with those: up to 736 keys, or 128-row workgroups for less than an eighth of the CUs.
 // waves: 0 chooses so; 4 or 12 fixes an unsplit layout (12 needs Lq >= 384); -3, -6 or -12 (that many waves, in three key
 // groups) a split one (more than 64 keys, Q's rows 16-byte aligned).
+// Past one round of twelve-wave workgroups, a last round that is nearly empty costs as much as a full one (B = 1, 24 heads x 9293
+// rows: 582 workgroups, 2.27 rounds). So whole rounds' worth of heads go to one twelve-wave launch, and the heads left over to a
+// second launch in whatever layout suits their number; only when that is twelve waves again do all heads stay in one launch.
+// One twelve-wave launch / four-wave / two launches, us: int8-QK 24 x 9293 1012 / 862 / 850, fp16 24 x 4200 314 / 252 / 228, 12 x 9000
+// 652 / 525 / 464, 24 x 6500 485 / 481 / 473. Two launches start and end twice: with few keys four waves are faster, to ~1300 keys fp16
+// (24 x 5000 by 1300: 111 / 91.2 / 90.6, by 800: 73.5 / 60.6 / 62.3) and ~2000 int8-QK (157 / 118.5 / 122). Where the last round is
+// at least two thirds full: four waves to ~700 and ~1400 keys (24 x 7500 by 700: 75.4 / 74.9, by 1300: 125.7 / 127.9; int8-QK 70.8 / 67.8
+// and 115.8 / 115.6).
 template <bool I8>
 static int launch_attn(AttnArgs a, int waves, void* stream) {
-    const long flat = (a.rows + FLAT_ROWS - 1) / FLAT_ROWS;
+    const long heads = a.rows / a.Lq_pad;
     // The split layouts need a tile for every key group, and copy Q's rows as K's and V's.
     const bool split = a.Lk > (SPLIT - 1) * KB && dma_ready(a.q, a.sqb, a.sqh, a.sql) && a.sql >= 0 && a.sql < (1L << 24);
-    if (waves == 0) {
-        int cus = 0;
-        if (const int e = device_cus(&cus)) return e;
-        const long heads = a.rows / a.Lq_pad;
-        auto grid = [&](int rows) { return heads * ((a.Lq + rows - 1) / rows); };
-        const bool few = split && a.Lk > 23 * KB && 8 * grid(QB) >= cus;
-        if (few && grid(32) <= cus) waves = -3;
-        else if (few && grid(64) <= cus) waves = -6;
-        else if (few && grid(QB) <= cus && (!I8 || a.Lk > 27 * KB)) waves = -12;
-        else waves = a.Lq >= FLAT_ROWS && 3 * flat >= 2L * cus ? 12 : 4;
+    const auto launch = [&](int waves, long first, long count) {
+        AttnArgs l = a;
+        l.head0 = (int)first;
+        l.rows = count * a.Lq_pad;
+        if (waves == 12 && a.Lq >= FLAT_ROWS) return launch_attn_layout<I8, 12, 1>(l, stream);
+        if (waves == 4) return launch_attn_layout<I8, 4, 1>(l, stream);
+        if (waves == -12 && split) return launch_attn_layout<I8, 4, SPLIT>(l, stream);
+        if (waves == -6 && split) return launch_attn_layout<I8, 2, SPLIT>(l, stream);
+        if (waves == -3 && split) return launch_attn_layout<I8, 1, SPLIT>(l, stream);
+        return RDA_ERR_INVALID;
+    };
+    if (waves != 0) return launch(waves, 0, heads);
+    int cus = 0;
+    if (const int e = device_cus(&cus)) return e;
+    const bool long_keys = a.Lk > 23 * KB;
+    const auto choose = [&](long heads, bool few) {
+        const auto grid = [&](int rows) { return heads * ((a.Lq + rows - 1) / rows); };
+        if (few && grid(32) <= cus) return -3;
+        if (few && grid(64) <= cus) return -6;
+        if (few && grid(QB) <= cus && (!I8 || a.Lk > 27 * KB)) return -12;
+        return a.Lq >= FLAT_ROWS && 3 * ((heads * a.Lq_pad + FLAT_ROWS - 1) / FLAT_ROWS) >= 2L * cus ? 12 : 4;
+    };
+    const long flat = (a.rows + FLAT_ROWS - 1) / FLAT_ROWS;
+    if (a.Lq >= FLAT_ROWS && flat > cus && flat % cus != 0) {
+        const long whole = flat / cus * cus * FLAT_ROWS / a.Lq_pad;  // the heads of whole rounds
+        const int rest = whole > 0 ? choose(heads - whole, split && long_keys) : 3 * (flat % cus) >= 2L * cus ? 12 : 4;
+        if (a.Lk <= (rest == 12 ? (I8 ? 44 : 24) : (I8 ? 64 : 40)) * KB) return launch(4, 0, heads);
+        if (rest != 12 && whole > 0) {
+            const int e = launch(12, 0, whole);
+            return e ? e : launch(rest, whole, heads - whole);
+        }
+        return launch(rest, 0, heads);
     }
-    if (waves == 12 && a.Lq >= FLAT_ROWS) return launch_attn_layout<I8, 12, 1>(a, stream);
-    if (waves == 4) return launch_attn_layout<I8, 4, 1>(a, stream);
-    if (waves == -12 && split) return launch_attn_layout<I8, 4, SPLIT>(a, stream);
-    if (waves == -6 && split) return launch_attn_layout<I8, 2, SPLIT>(a, stream);
-    if (waves == -3 && split) return launch_attn_layout<I8, 1, SPLIT>(a, stream);
-    return RDA_ERR_INVALID;
+    return launch(choose(heads, split && long_keys && 8 * heads * ((a.Lq + QB - 1) / QB) >= cus), 0, heads);
 }
-
 
 static bool attn_shapes_ok(int B, int H, int Hkv, int Lq, int Lk, const long* st) {
     const bool rows_ok = st[5] >= 0 && st[5] < (1L << 24) && st[8] >= 0 && st[8] < (1L << 24);

@@ -116,8 +116,9 @@ int rda_attn_i8(const void* q, const void* workspace, const void* v, void* out, 
  * (twelve-wave workgroups of 384 rows of the (batch, head, row) range; needs Lq >= 384), which give the same bits; -12, -6 or
  * -3 (workgroups of 128, 64 or 32 rows of one head, that many waves in three groups that share the keys out; Lk > 64, q's
  * rows 16-byte aligned), which give the same bits as each other; or 0 for the choice rda_attn makes (split keys from 737
- * keys on where a grid of 128-row workgroups has at most one per CU and at least one for every eighth CU; else twelve waves when Lq >= 384 and their grid covers
- * at least two thirds of the CUs; else four). No reference counterpart: for tests and measurement of each layout. Other
+ * keys on where a grid of 128-row workgroups has at most one per CU and at least one for every eighth CU; else twelve waves
+ * when Lq >= 384 and their grid covers at least two thirds of the CUs, the heads past its whole rounds in a second launch of
+ * another layout where that is faster; else four). No reference counterpart: for tests and measurement of each layout. Other
  * values return 1. */
 int rda_attn_waves(const void* q, const void* k, const void* v, void* out, int B, int H, int Hkv, int Lq, int Lk, const long* strides, float scale,
                    int waves, void* stream);
