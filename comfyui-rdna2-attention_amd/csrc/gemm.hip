@@ -839,10 +839,14 @@ constexpr TileCost I8_TILES[] = {
 constexpr TileCost I4_TILES[] = {
     {128, 256, 1, 6.03f, 0.52f, 0.73f, 0.f}, {128, 128, 2, 5.14f, 0.31f, 0.42f, 0.73f}, {64, 128, 2, 4.16f, 0.23f, 0.27f, 0.46f}, {64, 64, 2, 3.05f, 0.21f, 0.25f, 0.28f},
 };
-// The last one only where no other's staged group scales fit in LDS (K past ~31000).
+// The last one is built for one workgroup per CU: the staged group scales of the 128-column tiles above fit LDS up to K =
+// GROUP_WIDE_K only, and those of 64 x 64 up to 32000. Its constants are a fit to 154 shapes with K 1024-44416; for K past
+// GROUP_WIDE_K the rule then takes the faster of it and 64 x 64 on all 52 that both hold (4096 x 3072 x 16384 323 us against 360,
+// 1101 x 3072 x 16384 99 against 113, but 512 x 3072 x 16384 93 against 56). Below, it is never the fastest.
+#define GROUP_WIDE_K 15872
 constexpr TileCost GROUP_TILES[] = {
     {128, 128, 2, 5.25f, 0.54f, 0.70f, 1.18f}, {128, 256, 1, 5.90f, 0.86f, 1.17f, 0.f}, {64, 128, 2, 3.83f, 0.35f, 0.39f, 0.66f},
-    {64, 64, 2, 2.92f, 0.31f, 0.33f, 0.41f},   {128, 128, 1, 1e6f, 0.54f, 0.73f, 0.f},
+    {64, 64, 2, 2.92f, 0.31f, 0.33f, 0.41f},   {128, 128, 1, 3.20f, 0.69f, 0.77f, 0.f},
 };
 
 // Estimated us of an (M, N, K) product in tiles of t on 256 CUs: whole rounds of the workgroups the chip holds, then the
@@ -915,6 +919,7 @@ static int dispatch8(const void* a, const void* w, const float* as, const float*
         // in 128 x 256, 201.0 in 128 x 128, 231.7 in 64 x 128; 512 x 3072 x 12288: 38.0 in 64 x 128, 41.5 in 64 x 64, 60 before.
         if (group != 128 || K % 128 != 0 || !aligned(gs, 16)) return -1;
         if (IL && N % 128 != 0) return -1;
+        if (K <= GROUP_WIDE_K) tried = 1u << 4;
         for (int i; (i = best_tile(GROUP_TILES, tried, M, N, K)) >= 0;) {
             int e = -1;
             switch (i) {

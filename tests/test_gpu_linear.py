@@ -480,6 +480,24 @@ def test_group_scaled_tiles_bit_exact(dev, M, N, K):
     assert_same(bits(out), bits(oracle.w4a8_epilogue(oracle.w4a8_partials(q_ref, w.numpy()), s_ref, gs.numpy(), b.numpy())))
 
 
+# Past K = 15872 the tile is 64 x 64 or 128 x 128 with one workgroup per CU (past 32000 always the latter): many tiles take
+# 128 x 128, with N % 128 == 64 in natural order and a partial last column tile, else k-interleaved.
+@pytest.mark.parametrize("M,N,K,rotate", [(1101, 1984, 16384, True), (1101, 1920, 16384, True), (70, 192, 16384, True), (70, 320, 32768, False)])
+def test_group_scaled_long_rows_bit_exact(dev, M, N, K, rotate):
+    """The first and last rows and columns against the oracle (rows and columns are independent of each other)."""
+    print(f"group-scaled long rows M={M} N={N} K={K} rotate={rotate}", flush=True)
+    x = activations(M, K, seed=101, outliers=0)
+    w, wp = int4_weights(N, K, seed=102)
+    gs = (torch.rand(N, K // 128, generator=gen(103)) * 1.5e-2 + 5e-3).half()
+    b = (torch.randn(N, generator=gen(104)) * 0.5).half()
+    out = int8_gemm.linear_w4a8(x.to(dev), wp.to(dev), gs.to(dev), b.to(dev), rotate=rotate)
+    rows, cols = (np.r_[0:8, n - 35:n] for n in (M, N))
+    xr = x.numpy()[rows]
+    q_ref, s_ref = oracle.rot_quant_rows(xr)[:2] if rotate else oracle.quant_rows(xr)
+    ref = oracle.w4a8_epilogue(oracle.w4a8_partials(q_ref, w.numpy()[cols]), s_ref, gs.numpy()[cols], b.numpy()[cols])
+    assert_same(bits(out)[np.ix_(rows, cols)], bits(ref))
+
+
 def test_w4a4_hook_path_bit_exact(dev):
     """rot_quant_pack_a_i4 + gemm_i4 (the convrot_w4a4_forward replacement) against the oracle."""
     M, N, K = 600, 256, 1024
