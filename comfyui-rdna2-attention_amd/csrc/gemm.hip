@@ -386,6 +386,26 @@ __device__ __forceinline__ void epilogue_block(const i16v (&acc)[FI][FJ], const 
     }
 }
 
+// The order in which gemm8_kernel takes its gx x gy tiles: strips of `height` tile rows (the last one of `last`), `strip` tiles
+// each, with the factors that stand for the kernel's divisions: x / d = (x f) >> 32, f = ceil(2^32 / d), wherever
+// x (f d - 2^32) < 2^32 (tests/test_gemm_schedule.py). 0: no such factor (a divisor of 1, or a grid too large for it).
+struct TileOrder {
+    u32 strips, height, last, strip, per_strip, per_height, per_last;
+};
+static TileOrder tile_order(u32 gx, u32 gy, u32 most) {
+    auto factor = [](u32 d) { return d == 1 ? 0u : (u32)(((1ull << 32) + d - 1) / d); };
+    TileOrder o;
+    o.strips = (gy + most - 1) / most;
+    o.height = (gy + o.strips - 1) / o.strips;  // as even as they can be
+    o.last = gy - (o.strips - 1) * o.height;
+    o.strip = o.height * gx;
+    // A tile's number and f d - 2^32 are below gx gy and the strip's tiles; within a strip, below 2^29 and 8. A single strip: 0.
+    o.per_strip = o.strips == 1 ? 1 : (uint64_t)gx * gy * o.strip < 1ull << 32 ? factor(o.strip) : 0;
+    o.per_height = factor(o.height);
+    o.per_last = factor(o.last);
+    return o;
+}
+
 // int8 GEMM with direct global->LDS copies, for int8 or packed int4 weights (PER_CHANNEL, GROUP_SCALED and
 // RAW_ACC epilogues). A workgroup of NW wave64s (4 or 8) computes a BM x BN tile, the waves WGM x (NW / WGM)
 // over it (each a BM / WGM x BN / (NW / WGM) sub-tile: with four waves a BM/2 x BN/2 quarter, or with WGM = 1 all
@@ -420,7 +440,7 @@ template <int BM, int BN, int KB8, int NS, bool W4, int EPI, int MINB, int WGM, 
 __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, const float* __restrict__ as,
                                                       const float* __restrict__ ws, const half_t* __restrict__ gs, const half_t* __restrict__ bias,
                                                       void* __restrict__ Cout, int M, int N, int K, const half_t* __restrict__ R,
-                                                      const half_t* __restrict__ G, int L) {
+                                                      const half_t* __restrict__ G, int L, TileOrder order) {
     constexpr int NT = 64 * NW, WGN = NW / WGM, TM = BM / WGM, TN = BN / WGN, FI = TM / 32, FJ = TN / 32, NF = FI * FJ, NR = FI + FJ;
     constexpr bool GRP = EPI == GROUP_SCALED;
     constexpr int KS = KB8 / 32;                                      // 32-wide k steps per slice
@@ -442,15 +462,16 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
     // cover a nearly square part of C and read few A and W panels through its L2. Any grid: ids that go round-robin over the
     // columns instead have every XCD read every panel (int8, us in plain order -> strips: 2821 x 11136 x 1792 in 128 x 128 tiles
     // 86.2 -> 62.8, 533 x 5952 x 12032 59.6 -> 43.5, in 64 x 128 96.2 -> 57.8, 641 x 704 x 10496 in 64 x 64 18.8 -> 16.6). Strips about 1024 rows tall measured best
-    // of 1 to 16 tiles; the group-scaled 128-row tiles 4 tall (4096 x 12288 x 3072: 188.1 us against 190.3 at 8).
-    constexpr int STRIP = BM == 256 || GRP ? 4 : 8;
+    // of 1 to 16 tiles; the group-scaled 128-row tiles 4 tall (4096 x 12288 x 3072: 188.1 us against 190.3 at 8). The strips come from
+    // the launcher (tile_order): divided out here, they held back each workgroup's first copy by @@.
     int bx, by;
     {
-        const int gx = gridDim.x, gy = gridDim.y, n = gx * gy, id = blockIdx.y * gx + blockIdx.x, x = id % 8;
-        const int strips = (gy + STRIP - 1) / STRIP, height = (gy + strips - 1) / strips;  // as even as they can be
-        const int s = x * (n / 8) + min(x, n % 8) + id / 8, strip = s / (height * gx), w = s - strip * height * gx, tall = min(height, gy - strip * height);
-        bx = w / tall;
-        by = strip * height + w - bx * tall;
+        const u32 n = gridDim.x * gridDim.y, id = blockIdx.y * gridDim.x + blockIdx.x, x = id % 8;
+        const u32 s = x * (n / 8) + min(x, n % 8) + id / 8, strip = order.per_strip ? __umulhi(s, order.per_strip) : s / order.strip;
+        const u32 w = s - strip * order.strip, per = strip == order.strips - 1 ? order.per_last : order.per_height;
+        const u32 tall = strip == order.strips - 1 ? order.last : order.height;
+        bx = (int)(per ? __umulhi(w, per) : w);
+        by = (int)(strip * order.height + w - bx * tall);
     }
     const int m0 = by * BM, n0 = bx * BN;
     const int wrow = W4 ? K / 2 : K;  // bytes per W row in memory
@@ -813,8 +834,10 @@ static int launch_gemm8(const void* a, const void* w, const float* as, const flo
     auto kern = gemm8_kernel<BM, BN, KB8, NS, W4, EPI, MINB, WGM, NW, IL, RA>;
     static std::atomic<size_t> configured[RDA_MAX_DEVICES];
     if (const int e = ensure_dynamic_lds((const void*)kern, lds, configured)) return e;
-    hipLaunchKernelGGL(kern, dim3((N + BN - 1) / BN, (M + BM - 1) / BM), dim3(64 * NW), lds, (hipStream_t)stream, (const int8_t*)a, (const int8_t*)w, as, ws,
-                       (const half_t*)gs, (const half_t*)bias, c, M, N, K, (const half_t*)R, (const half_t*)G, L);
+    const int gx = (N + BN - 1) / BN, gy = (M + BM - 1) / BM;
+    constexpr int STRIP = BM == 256 || EPI == GROUP_SCALED ? 4 : 8;
+    hipLaunchKernelGGL(kern, dim3(gx, gy), dim3(64 * NW), lds, (hipStream_t)stream, (const int8_t*)a, (const int8_t*)w, as, ws, (const half_t*)gs,
+                       (const half_t*)bias, c, M, N, K, (const half_t*)R, (const half_t*)G, L, tile_order(gx, gy, STRIP));
     return (int)hipGetLastError();
 }
 

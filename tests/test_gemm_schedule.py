@@ -259,6 +259,54 @@ def tile_of(block, gx, gy, strips):
     return w // h, strip * tall + w % h
 
 
+def tile_order(gx, gy, most):
+    """tile_order in csrc/gemm.hip: the strips, and the factors that stand for divisions (0: none)."""
+    factor = lambda d: 0 if d == 1 else -(-2**32 // d)  # noqa: E731
+    strips = -(-gy // most)
+    height = -(-gy // strips)
+    last, strip = gy - (strips - 1) * height, height * gx
+    per_strip = 1 if strips == 1 else factor(strip) if gx * gy * strip < 2**32 else 0
+    return strips, height, last, strip, per_strip, factor(height), factor(last)
+
+
+def tile_by_factors(s, order):
+    """The kernel's steps from a tile's number in the order of strips to (bx, by), in 32-bit arithmetic."""
+    strips, height, last, strip_tiles, per_strip, per_height, per_last = order
+    strip = s * per_strip >> 32 if per_strip else s // strip_tiles
+    w = s - strip * strip_tiles
+    per, tall = (per_last, last) if strip == strips - 1 else (per_height, height)
+    assert max(order) < 2**32 and 0 <= w < 2**32
+    bx = w * per >> 32 if per else w
+    return bx, strip * height + w - bx * tall
+
+
+@pytest.mark.parametrize("most", [4, 8])
+@pytest.mark.parametrize("gx,gy", [(1, 1), (1, 9), (7, 1), (3, 17), (48, 32), (87, 23), (12, 16), (192, 128), (5, 1000), (3000, 33), (48, 5000), (1, 250000), (200000, 7),
+                                   (60000, 3001)])
+def test_tile_order_factors_divide_exactly(gx, gy, most):
+    """Every tile of a small grid and, in a large one, the tiles around each strip's and column's edge: what the factors give is what
+    dividing gives, up to the largest grids (60000 x 3001 is past the strip factor's range and divides)."""
+    order = tile_order(gx, gy, most)
+    strips, height, last, strip_tiles = order[:4]
+    n = gx * gy
+    assert strips * most >= gy and 1 <= last <= height <= most and (strips - 1) * height + last == gy
+    numbers = range(n) if n < 30000 else sorted({min(max(e + d, 0), n - 1) for k in {0, 1, 2, strips // 2, strips - 2, strips - 1} for c in (0, 1, 2, gx // 2, gx - 1)
+                                                 for e in (k * strip_tiles, k * strip_tiles + c * height, k * strip_tiles + c * last) for d in (-1, 0, 1)})
+    for s in numbers:
+        strip, w = divmod(s, strip_tiles)
+        tall = min(height, gy - strip * height)
+        assert tile_by_factors(s, order) == (w // tall, strip * height + w % tall)
+
+
+def test_strip_factor_needs_its_range():
+    order = tile_order(59990, 3001, 8)
+    assert order[4] == 0
+    number, taken = (order[0] - 1) * order[3] - 1, (*order[:4], -(-2**32 // order[3]), *order[5:])  # a strip's last tile; the factor all the same
+    assert tile_by_factors(number, order) == ((order[3] - 1) // order[1], (order[0] - 1) * order[1] - 1)
+    with pytest.raises(AssertionError):
+        tile_by_factors(number, taken)
+
+
 @pytest.mark.parametrize("strips", [False, True])
 @pytest.mark.parametrize("gx,gy", [(48, 32), (24, 9), (1, 1), (3, 17), (87, 23), (12, 16), (16, 16), (4, 8), (8, 4), (96, 32), (6, 3), (5, 8)])
 def test_tile_order_is_a_permutation(gx, gy, strips):
