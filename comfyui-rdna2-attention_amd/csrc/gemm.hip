@@ -301,7 +301,7 @@ __device__ __forceinline__ void epilogue_rows(const i16v (&acc)[FI][FJ], int lan
 // 128-byte lines (the register layout would touch 32 rows per instruction). R and G are read the same way.
 // Bytes of the bias area of the scale block: BN halfs, copied in 256-byte instructions.
 constexpr int SC_BIAS(int bn) { return (bn * 2 + 255) / 256 * 256; }
-template <int BM, int BN, int FI, int FJ, int EPI, int NT>
+template <int BM, int BN, int FI, int FJ, int EPI, int NT, bool WHOLE>  // WHOLE: every column tile is (N a multiple of BN)
 __device__ __forceinline__ void epilogue_block(const i16v (&acc)[FI][FJ], const f16v (&yacc)[EPI == GROUP_SCALED ? FI : 1][EPI == GROUP_SCALED ? FJ : 1],
                                                char* tile, const char* sc, int t, int lane, int wm, int wn, int m0, int n0, int M, int N,
                                                const float* __restrict__ as, const float* __restrict__ ws, const half_t* __restrict__ bias,
@@ -340,15 +340,22 @@ __device__ __forceinline__ void epilogue_block(const i16v (&acc)[FI][FJ], const 
     };
     constexpr int ITER = BM * CPR / NT;  // 16-byte chunks per thread (the tile is a whole number of them)
     static_assert(BM * CPR % NT == 0, "whole chunks per thread");
+    // With 24 chunks per row a thread's column changes from chunk to chunk, and its check costs 0.2-0.3 us of a 256 x 192 tile
+    // (873 x 2880 x 192 9.1 us with both, 8.7 without either): only in tiles that need it.
+    const bool all = WHOLE || (NT % CPR != 0 && n0 + BN <= N);
     if (!R) {
         if (bias) dequantize(std::integral_constant<bool, true>{});
         else dequantize(std::integral_constant<bool, false>{});
         __syncthreads();
+        auto rows = [&](auto all_columns) __attribute__((always_inline)) {
 #pragma unroll 4
-        for (int it = 0; it < ITER; it++) {
-            const int idx = t + it * NT, r = idx / CPR, c = (idx % CPR) * 8, m = m0 + r;
-            if (m < M && n0 + c < N) *(h8*)(C + (size_t)m * N + n0 + c) = *(const h8*)(tile + r * TP + c * 2);
-        }
+            for (int it = 0; it < ITER; it++) {
+                const int idx = t + it * NT, r = idx / CPR, c = (idx % CPR) * 8, m = m0 + r;
+                if (m < M && (decltype(all_columns)::value || n0 + c < N)) *(h8*)(C + (size_t)m * N + n0 + c) = *(const h8*)(tile + r * TP + c * 2);
+            }
+        };
+        if (all) rows(std::integral_constant<bool, true>{});
+        else rows(std::integral_constant<bool, false>{});
         return;
     }
     // Gated residual: R and G are read in batches of RB chunks per thread, double-buffered, with row indices
@@ -359,31 +366,36 @@ __device__ __forceinline__ void epilogue_block(const i16v (&acc)[FI][FJ], const 
     // 64 x 128 (128 accumulator VGPRs of a 256 budget) take batches of 4.
     constexpr int RBMAX = NT >= 512 && FI * FJ >= 8 ? 4 : 8;
     constexpr int RB = ITER % RBMAX == 0 ? RBMAX : ITER % 4 == 0 ? 4 : 1, NBATCH = ITER / RB;
-    h8 res[2][RB], gat[2][RB];
-    auto load = [&](int b, int slot) __attribute__((always_inline)) {
+    auto gated = [&](auto all_columns) __attribute__((always_inline)) {
+        constexpr bool ALL = decltype(all_columns)::value;
+        h8 res[2][RB], gat[2][RB];
+        auto load = [&](int b, int slot) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < RB; k++) {
-            const int idx = t + (b * RB + k) * NT, r = idx / CPR, n = min(n0 + (idx % CPR) * 8, N - 8), m = min(m0 + r, M - 1);
-            res[slot][k] = *(const h8*)(R + (size_t)m * N + n);
-            gat[slot][k] = *(const h8*)(G + (size_t)(m / L) * N + n);
+            for (int k = 0; k < RB; k++) {
+                const int idx = t + (b * RB + k) * NT, r = idx / CPR, c = n0 + (idx % CPR) * 8, n = ALL ? c : min(c, N - 8), m = min(m0 + r, M - 1);
+                res[slot][k] = *(const h8*)(R + (size_t)m * N + n);
+                gat[slot][k] = *(const h8*)(G + (size_t)(m / L) * N + n);
+            }
+        };
+        load(0, 0);
+        if (bias) dequantize(std::integral_constant<bool, true>{});
+        else dequantize(std::integral_constant<bool, false>{});
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NBATCH; b++) {
+            if (b + 1 < NBATCH) load(b + 1, (b + 1) & 1);
+#pragma unroll
+            for (int k = 0; k < RB; k++) {
+                const int idx = t + (b * RB + k) * NT, r = idx / CPR, c = (idx % CPR) * 8, m = m0 + r;
+                h8 y = *(const h8*)(tile + r * TP + c * 2);
+#pragma unroll
+                for (int e = 0; e < 8; e++) y[e] = to_half((float)res[b & 1][k][e] + r16((float)gat[b & 1][k][e] * (float)y[e]));
+                if (m < M && (ALL || n0 + c < N)) *(h8*)(C + (size_t)m * N + n0 + c) = y;
+            }
         }
     };
-    load(0, 0);
-    if (bias) dequantize(std::integral_constant<bool, true>{});
-    else dequantize(std::integral_constant<bool, false>{});
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < NBATCH; b++) {
-        if (b + 1 < NBATCH) load(b + 1, (b + 1) & 1);
-#pragma unroll
-        for (int k = 0; k < RB; k++) {
-            const int idx = t + (b * RB + k) * NT, r = idx / CPR, c = (idx % CPR) * 8, m = m0 + r;
-            h8 y = *(const h8*)(tile + r * TP + c * 2);
-#pragma unroll
-            for (int e = 0; e < 8; e++) y[e] = to_half((float)res[b & 1][k][e] + r16((float)gat[b & 1][k][e] * (float)y[e]));
-            if (m < M && n0 + c < N) *(h8*)(C + (size_t)m * N + n0 + c) = y;
-        }
-    }
+    if (all) gated(std::integral_constant<bool, true>{});
+    else gated(std::integral_constant<bool, false>{});
 }
 
 // The order in which gemm8_kernel takes its gx x gy tiles: strips of `height` tile rows (the last one of `last`), `strip` tiles
@@ -819,7 +831,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
         epilogue_rows<FI, FJ, EPI>(acc, lane, m0 + wm * TM, n0 + wn * TN, M, N, as, ws, bias, Cout, R, G, L);
     } else {
         __syncthreads();  // the staged tile overlaps the stages
-        epilogue_block<BM, BN, FI, FJ, EPI, NT>(acc, yacc, smem, sc, t, lane, wm, wn, m0, n0, M, N, as, ws, bias, (half_t*)Cout, R, G, L);
+        epilogue_block<BM, BN, FI, FJ, EPI, NT, KB8 == 64>(acc, yacc, smem, sc, t, lane, wm, wn, m0, n0, M, N, as, ws, bias, (half_t*)Cout, R, G, L);
     }
 }
 
