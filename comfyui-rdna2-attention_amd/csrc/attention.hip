@@ -124,7 +124,10 @@ __global__ __launch_bounds__(64 * NR * NS) __attribute__((amdgpu_waves_per_eu(NR
     constexpr int KS = NSET * T::K_BYTES, VS = NSET * T::V_BYTES, VOFF = 3 * KS;
     const int t = threadIdx.x, lane = t & 63, g = lane >> 5, lq = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // scalar
-    const int grp = wave / NR, wq = wave % NR;                 // key group, and wave of it
+    // Key group, and wave of it. The compiler does not see that a four-wave workgroup has one group, and carried it through the tile
+    // loop: 2 heads x 39 rows by 2464 keys (one wave per SIMD) 42.8 us, 41.6 with the constant, 4 x 300 by 9000 149.9 / 144.6. (Twelve waves
+    // measured 0.5% slower with it.)
+    const int grp = NS > 1 || FLAT ? wave / NR : 0, wq = wave % NR;
 
     // Block remap: consecutive block ids go round-robin to the 8 XCDs; give each XCD a contiguous run
     // of (head, q-block) work so its resident workgroups share K/V through its L2 (the first XCDs one more block each
