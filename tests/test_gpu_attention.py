@@ -127,6 +127,88 @@ def test_attention_choice_of_layout(dev, int8_qk, B, H, Lq, Lk):
         close(views[1][:, heads][:, :, rows.to(dev)], ref)
 
 
+def softmax_state_inputs(kind, B, H, Lq, Lk):
+    """q, k, v whose running maxima move: scores far above the rescale bound, climbing along the keys, zero query rows, or the largest
+    scores in the tiles of one key group (32-key tiles j, j + 3, ...) only, tens of log2 units above the others."""
+    q, k, v = qkv(B, H, H, Lq, Lk, seed=Lk + Lq)
+    tile = torch.arange(Lk) // 32
+    if kind == "large":
+        q = (q.float() * 4).half()
+    elif kind == "rising":
+        q = (torch.rand(B, H, Lq, 128, generator=gen(21)) * 0.5 + 0.5).half()
+        k = (torch.linspace(0.0, 8.0, Lk).view(1, 1, Lk, 1) + k.float() * 0.05).half()
+    elif kind == "zero rows":
+        q[:, :, ::3] = 0
+    else:
+        q = (q.float() * 2).half()
+        k = (k.float() * torch.where(tile % 3 == int(kind[-1]), 4.0, 0.25).view(1, 1, Lk, 1)).half()
+    return q, k, v
+
+
+# 27 tiles (nine per group), 37 and a last one of a single key (groups 0 and 1 a tile more than group 2, the single key in group 1),
+# and three tiles, of which group 2's is the single key.
+@pytest.mark.parametrize("Lk", [864, 1185, 65])
+@pytest.mark.parametrize("kind", ["large", "rising", "zero rows", "group 0", "group 1", "group 2"])
+@pytest.mark.parametrize("int8_qk", [False, True])
+def test_attention_split_keys_softmax_states(dev, int8_qk, kind, Lk):
+    """The rescale inside a key group and the merge of groups whose maxima differ, each split layout against the float64 closed form
+    and bit for bit equal to the others (the unsplit one beside them)."""
+    print(f"split keys, softmax states {kind} Lk={Lk} int8_qk={int8_qk}", flush=True)
+    q, k, v = softmax_state_inputs(kind, 1, 2, 150, Lk)
+    ref = (oracle.attention_i8qk_f64 if int8_qk else oracle.attention_f64)(q.numpy(), k.numpy(), v.numpy(), 128 ** -0.5)
+    outs = [attention_layout(q.to(dev), k.to(dev), v.to(dev), 128 ** -0.5, int8_qk, waves) for waves in (4, -12, -6, -3)]
+    for out in outs:
+        close(out, ref)
+    for out in outs[2:]:
+        assert torch.equal(out.view(torch.int16), outs[1].view(torch.int16))
+
+
+def test_attention_split_keys_non_finite(dev):
+    """A group whose scores are all -inf drops out of the merge; a NaN key makes every row NaN, an infinite value its column infinite,
+    in every layout."""
+    q, k, v = qkv(1, 2, 2, 100, 300, seed=31)
+    q = q.abs() + 0.01  # positive, so that a key of -inf scores -inf
+    for group in range(3):
+        dead = torch.arange(300) // 32 % 3 == group
+        kd = k.clone()
+        kd[:, :, dead] = -math.inf
+        ref = oracle.attention_f64(q.numpy(), k[:, :, ~dead].numpy(), v[:, :, ~dead].numpy(), 128 ** -0.5)
+        for waves in (4, -12, -6, -3):
+            print(f"-inf scores in group {group}, waves {waves}", flush=True)
+            close(attention_layout(q.to(dev), kd.to(dev), v.to(dev), 128 ** -0.5, False, waves), ref)
+    kn, vi = k.clone(), v.clone()
+    kn[0, 0, 45] = math.nan  # group 1
+    vi[0, 1, 70, 5] = math.inf  # group 2
+    for waves in (4, -12, -6, -3):
+        print(f"NaN key and infinite value, waves {waves}", flush=True)
+        out = attention_layout(q.to(dev), kn.to(dev), vi.to(dev), 128 ** -0.5, False, waves).cpu()
+        assert out[0, 0].isnan().all() and (out[0, 1, :, 5] == math.inf).all()
+        out[0, 1, :, 5] = 0
+        assert out[0, 1].isfinite().all()
+
+
+@pytest.mark.parametrize("int8_qk,Lk", [(False, 1500), (True, 2100)])
+def test_attention_two_launches_softmax_states(dev, int8_qk, Lk):
+    """60 heads x 1800 rows: 53 heads in whole rounds of twelve-wave workgroups, the others in a second launch with split keys.
+    Climbing scores, large scores and zero rows in different heads; a second call gives the same bits."""
+    print(f"two launches, softmax states Lk={Lk} int8_qk={int8_qk}", flush=True)
+    B, H, Lq = 1, 60, 1800
+    kinds = {0: "large", 52: "rising", 53: "rising", 54: "zero rows", 57: "group 1", 59: "large"}
+    q, k, v = qkv(B, H, H, Lq, Lk, seed=33)
+    for h, kind in kinds.items():
+        for t, one in zip((q, k, v), softmax_state_inputs(kind, 1, 1, Lq, Lk)):
+            t[:, h] = one[:, 0]
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    outs = [torch.empty(B, H, Lq, 128, dtype=torch.float16, device=dev) for _ in range(2)]
+    for out in outs:
+        hip_attention.attention(qd, kd, vd, out, 128 ** -0.5, int8_qk)
+    assert torch.equal(*(out.view(torch.int16) for out in outs))
+    rows = torch.cat([torch.arange(0, 33), torch.arange(Lq - 33, Lq)])
+    heads = list(kinds)
+    ref = (oracle.attention_i8qk_f64 if int8_qk else oracle.attention_f64)(q[:, heads][:, :, rows].numpy(), k[:, heads].numpy(), v[:, heads].numpy(), 128 ** -0.5)
+    close(outs[0][:, heads][:, :, rows.to(dev)], ref)
+
+
 @pytest.mark.parametrize("int8_qk", [False, True])
 def test_attention_zero_query_rows(dev, int8_qk):
     """All-zero query rows (the int8 row scale then sits at its 1e-30 floor) with a partial last key tile: the keys past
