@@ -334,9 +334,8 @@ def test_swiglu_down_linear_bit_exact(dev, M, K, N):
     assert_same(bits(out), bits(ref))
 
 
-# K / 128 = 8, 4, 24 and 26 slices: whole and partial passes of the slice loop over the three stages; 2, 6 and 10 slices
-# (tail slices only; one pass and its tail); K = 12288 and 8192 (past K = 3456 the block's group scales no longer fit
-# two blocks per CU: one block per CU)
+# K / 128 = 8, 4, 24 and 26 slices: whole and partial passes of the slice loop over the stages; 2, 6 and 10 slices (tail slices
+# only; one pass and its tail); K = 12288 and 8192 (many group scales staged)
 @pytest.mark.parametrize("M,N,K", [(520, 512, 1024), (300, 192, 512), (4096, 1024, 3072), (200, 256, 3328), (520, 256, 12288), (300, 384, 8192),
                                    (64, 128, 256), (200, 256, 768), (129, 128, 1280)])
 def test_w4a8_bit_exact(dev, M, N, K):
@@ -390,8 +389,8 @@ def test_w4a8_full_size_every_output(dev):
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), f"{(out != ref).sum().item()} outputs differ"
 
 
-# Shapes of each block the k-interleaved pair runs (two 128 x 128 blocks per CU; past K = 3456 one 128 x 256 block, or
-# one 128 x 128 block when N % 256 != 0), rotation groups 256 and 128, a partial last row block, with and without bias.
+# The k-interleaved pair in 64 x 64 tiles (the rule's choice for few tiles; test_group_scaled_tiles_bit_exact, test_w4a8_full_size_*
+# and test_group_scaled_long_rows_bit_exact run the others), rotation groups 256 and 128, a partial last row tile, with and without bias.
 @pytest.mark.parametrize("M,N,K,group,with_bias", [(520, 512, 1024, 256, False), (200, 256, 12288, 256, True), (300, 384, 8192, 128, False),
                                                    (129, 128, 1280, 256, True), (64, 128, 128, 128, False)])
 def test_w4a8_interleaved_pair_matches_natural(dev, M, N, K, group, with_bias):
@@ -466,10 +465,10 @@ def test_int4_tiles_bit_exact(dev, M, N, K):
     assert_same(bits(out), bits(oracle.gemm_epilogue(oracle.gemm_acc(q_ref, w.numpy()), s_ref, ws.numpy())))
 
 
-@pytest.mark.parametrize("M,N,K", [(5, 64, 384), (659, 3008, 128), (4110, 960, 128), (1863, 2240, 640), (1666, 1280, 640), (70, 256, 12288)])
+@pytest.mark.parametrize("M,N,K", [(5, 64, 384), (659, 3008, 128), (4110, 960, 128), (1863, 2240, 640), (1666, 1280, 640), (70, 256, 12288), (1863, 2304, 640)])
 def test_group_scaled_tiles_bit_exact(dev, M, N, K):
     """W4A8 in 64 x 64, 64 x 128, 128 x 128 and 128 x 256 tiles with partial last tiles, in natural order (N % 128 == 64),
-    then k-interleaved 64 x 128 and 64 x 64 tiles."""
+    then k-interleaved 64 x 128, 64 x 64 and 128 x 256 tiles."""
     print(f"group-scaled tiles M={M} N={N} K={K}", flush=True)
     x = activations(M, K, seed=95, outliers=0)
     w, wp = int4_weights(N, K, seed=96)
@@ -531,6 +530,73 @@ def test_w8a8_linear_unaligned_weight_view(dev):
     out = int8_gemm.linear(x.to(dev), wu, ws.to(dev), None, rotate=True)
     q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy())
     assert_same(bits(out), bits(oracle.gemm_epilogue(oracle.gemm_acc(q_ref, w.numpy()), s_ref, ws.numpy())))
+
+
+def unaligned(t, dev):
+    """t on the GPU, 4 bytes into its storage."""
+    buf = torch.empty(t.numel() + 4, dtype=t.dtype, device=dev)
+    view = buf[4 // t.element_size():][:t.numel()].view(t.shape)
+    assert view.copy_(t.to(dev)).data_ptr() % 16 == 4
+    return view
+
+
+# The register-load GEMM's tiles are 256 rows by 64, 128 and 256 columns (N = 64 and 320, 128, 256); M = 300 leaves the last one partial.
+@pytest.mark.parametrize("epilogue", ["bias", "residual"])
+@pytest.mark.parametrize("N", [64, 128, 256, 320])
+def test_register_load_gemm_bit_exact(dev, N, epilogue):
+    """int8 weights the direct-copy kernel cannot read (unaligned), with a bias or the gated residual, and as raw accumulators."""
+    print(f"register-load GEMM N={N} {epilogue}", flush=True)
+    B, L, K = 2, 150, 512
+    x, w, ws = activations(B * L, K, seed=111), int8_weights(N, K, seed=112), channel_scales(N, seed=113)
+    q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy())
+    acc, wu = oracle.gemm_acc(q_ref, w.numpy()), unaligned(w, dev)
+    if epilogue == "bias":
+        b = (torch.randn(N, generator=gen(114)) * 0.5).half()
+        out = int8_gemm.linear(x.to(dev), wu, ws.to(dev), b.to(dev), rotate=True)
+        ref = oracle.gemm_epilogue(acc, s_ref, ws.numpy(), b.numpy())
+        packed, _ = int8_gemm.quantize(kern().rot_quant_pack_a, x.to(dev), K)
+        assert torch.equal(int8_gemm.gemm_acc(packed, wu, B * L, K).cpu(), torch.from_numpy(acc))
+    else:
+        R, G = torch.randn(B, L, N, generator=gen(115)).half(), torch.randn(B, N, generator=gen(116)).half()
+        out = int8_gemm.linear(x.to(dev), wu, ws.to(dev), None, rotate=True, res=(R.to(dev), G.to(dev)))
+        ref = oracle.gemm_epilogue(acc, s_ref, ws.numpy(), R=R.numpy().reshape(B * L, N), G=G.numpy(), L=L)
+    assert_same(bits(out), bits(ref))
+
+
+@pytest.mark.parametrize("N", [64, 128, 256, 320])
+def test_register_load_gemm_int4_bit_exact(dev, N):
+    """Packed int4 weights that are not 16-byte aligned: W4A4, and W4A8 with a bias (tiles of 128 x 256 and 256 x 64)."""
+    print(f"register-load int4 GEMM N={N}", flush=True)
+    M, K = 300, 512
+    x, ws = activations(M, K, seed=121), channel_scales(N, seed=123)
+    w, wp = int4_weights(N, K, seed=122)
+    wu, k = unaligned(wp, dev), kern()
+    out = int8_gemm.run(k.rot_quant_pack_a_i4, k.gemm_i4, x.to(dev), wu, ws.to(dev), None, K)
+    q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), i4=True)
+    assert_same(bits(out), bits(oracle.gemm_epilogue(oracle.gemm_acc(q_ref, w.numpy()), s_ref, ws.numpy())))
+    gs = (torch.rand(N, K // 128, generator=gen(124)) * 1.5e-2 + 5e-3).half()
+    b = (torch.randn(N, generator=gen(125)) * 0.5).half()
+    out = int8_gemm.linear_w4a8(x.to(dev), wu, gs.to(dev), b.to(dev))
+    q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy())
+    assert_same(bits(out), bits(oracle.w4a8_epilogue(oracle.w4a8_partials(q_ref, w.numpy()), s_ref, gs.numpy(), b.numpy())))
+
+
+# K % 128 == 64: 64-value slices, in 256-row tiles of 256, 192 or 128 columns where one divides N (three and seven slices for four
+# stages), else the register-load GEMM.
+@pytest.mark.parametrize("K", [192, 448])
+@pytest.mark.parametrize("N", [64, 128, 192, 256, 320])
+def test_half_slices_bit_exact(dev, N, K):
+    print(f"half slices N={N} K={K}", flush=True)
+    B, L = 2, 139
+    x, w, ws = activations(B * L, K, seed=131), int8_weights(N, K, seed=132), channel_scales(N, seed=133)
+    b = (torch.randn(N, generator=gen(134)) * 0.5).half()
+    R, G = torch.randn(B, L, N, generator=gen(135)).half(), torch.randn(B, N, generator=gen(136)).half()
+    q_ref, s_ref = oracle.quant_rows(x.numpy())
+    acc = oracle.gemm_acc(q_ref, w.numpy())
+    out = int8_gemm.linear(x.to(dev), w.to(dev), ws.to(dev), b.to(dev))
+    assert_same(bits(out), bits(oracle.gemm_epilogue(acc, s_ref, ws.numpy(), b.numpy())))
+    out = int8_gemm.linear(x.to(dev), w.to(dev), ws.to(dev), None, res=(R.to(dev), G.to(dev)))
+    assert_same(bits(out), bits(oracle.gemm_epilogue(acc, s_ref, ws.numpy(), R=R.numpy().reshape(B * L, N), G=G.numpy(), L=L)))
 
 
 def test_plain_int8_linear_long_rows(dev):
