@@ -1,5 +1,7 @@
 """Parity of the linear path on the GPU (through the C ABI) against the oracle: quantized activations and scales
 bit-exact, int32 accumulators bit-exact, fp16 outputs bit-exact (the epilogue is IEEE fp32 in a fixed order)."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -139,6 +141,51 @@ def test_quantizer_row_ranges_bit_exact(dev, kind, K, group):
         q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), group=group, i4=True)
     assert_same(scale.cpu().numpy(), s_ref)
     assert_same(q_of(packed, M, K), q_ref)
+
+
+@pytest.mark.parametrize("kind,K,group", [(kind, 1280, 256) for kind in ("plain", "rot", "il", "int4", "swiglu", "gate", "situ", "mod")]
+                         + [(kind, 640, 128) for kind in ("rot", "il", "int4", "swiglu", "gate", "situ")])
+def test_quantizers_non_finite_rows(dev, kind, K, group):
+    """NaN, infinities and the largest fp16 values in one place of a row or all along it, in either operand: scales and codes are the
+    oracle's (a NaN is the lowest code and no maximum). A row of infinite scale has no finite quotient: all its codes are the lowest."""
+    print(f"non-finite rows {kind} K={K} group={group}", flush=True)
+    k, g = kern(), gen(K)
+    x, u = torch.randn(16, K, generator=g).half(), torch.randn(16, K, generator=g).half()
+    specials = torch.tensor([math.nan, math.inf, -math.inf, 65504.0, -65504.0, 0.0]).half()
+    for i, v in enumerate(specials):
+        x[i, 37 * i] = v
+        x[6 + i] = v
+    u[12, 5], u[13, 9], u[14, 11], u[15] = math.nan, math.inf, -math.inf, math.inf
+    xd, ud = x.to(dev), u.to(dev)
+    if kind == "plain":
+        packed, scale = int8_gemm.quantize(k.quant_pack_a, xd, K)
+        q_ref, s_ref = oracle.quant_rows(x.numpy())
+    elif kind in ("rot", "il", "int4"):
+        entry = {"rot": k.rot_quant_pack_a, "il": k.rot_quant_pack_a_il, "int4": k.rot_quant_pack_a_i4}[kind]
+        packed, scale = int8_gemm.quantize(entry, xd, K, group=group)
+        q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), group=group, i4=kind == "int4")
+    elif kind == "situ":
+        both = torch.cat([x, u], 1)
+        packed, scale = int8_gemm.quantize(k.situ_rot_quant_pack_a, both.to(dev), K, group=group)
+        q_ref, s_ref, _ = oracle.rot_quant_rows(both.numpy(), act=oracle.ACT_SITU, group=group)
+    elif kind == "mod":
+        w, s, t = torch.randn(K, generator=g) * 0.1, torch.randn(1, K, generator=g).half(), torch.randn(1, K, generator=g).half()
+        packed, scale = int8_gemm.quantized(16, K, dev)
+        p, (wd, sd, td) = _lib.ptr, (v.to(dev) for v in (w, s, t))
+        _lib.call("rda_mod_rot_quant_pack_a", p(xd), p(packed), p(scale), 16, K, p(wd), p(sd), p(td), 16, 1e-6)
+        q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), act=oracle.ACT_MOD, mod=(w.numpy(), s.numpy(), t.numpy(), 16, 1e-6))
+    else:
+        act = oracle.ACT_SWIGLU if kind == "swiglu" else oracle.ACT_GATE
+        entry = k.swiglu_rot_quant_pack_a if kind == "swiglu" else k.gate_rot_quant_pack_a
+        packed, scale = int8_gemm.quantize(entry, xd, K, up=ud, group=group)
+        q_ref, s_ref, _ = oracle.rot_quant_rows(x.numpy(), act=act, group=group, u=u.numpy())
+    q = q_of(packed, 16, K)
+    if kind == "il":
+        q = q.reshape(16, K // 8, 2, 4).swapaxes(2, 3).reshape(16, K)
+    assert_same(scale.cpu().numpy(), s_ref)
+    infinite = np.isinf(s_ref)
+    assert_same(q[~infinite], q_ref[~infinite])
+    assert (q[infinite] == (-7 if kind == "int4" else -128)).all()
 
 
 @pytest.mark.parametrize("B,L,K", [(1, 77, 3072), (2, 40, 1024)])
