@@ -326,7 +326,7 @@ __global__ __launch_bounds__(64 * NR * NS) __attribute__((amdgpu_waves_per_eu(NR
     float m = -1e30f, l = 0.f;
 
     // LDS offsets of the lane's V^T reads (and int8 K reads) within a stage, fixed for the whole loop: the stage
-    // enters as an immediate offset (the loop below is unrolled over the two stages), so the tile loop spends
+    // enters as an immediate offset (the loop below is unrolled over the three stages), so the tile loop spends
     // no VALU on them. Kept opaque so that the compiler holds them in VGPRs rather than recomputing them.
     u32 k_rd[4];
     u32 ks_rd = 0;

@@ -444,10 +444,11 @@ static TileOrder tile_order(u32 gx, u32 gy, u32 most) {
 // (sched_barrier pins the order). Fragments are read RA k steps ahead; the slice's barrier sits before its last
 // RA k steps, so the next slice's first reads start right after it. RA 1 for the 256-row tiles, whose k step holds 6 or 8
 // products per wave, enough to cover an LDS read; RA 3 (a slice's fragments in registers before its products) for
-// the smaller ones, whose 1 to 6 products do not: 64 x 128, 512 x 3072 x 3072 11.1 -> 9.9 us; 128 x 128, 1101 x 3072 x 8192 33.7 ->
-// 30.4. What bounds the small tiles then is their copies, ~100 GB/s per CU (64 x 64: 0.16 us per 16 KiB slice);
-// more stages (6 to 8) measured slower, as did a k start that differs by block. The 256-row tiles are bound by power:
-// 4096 x 3072 x 3072 takes 28.7 us on zeros and 37-43 on random operands, whatever the tile.
+// the smaller ones, whose 1 to 6 products do not: 64 x 128, 512 x 3072 x 3072 11.1 -> 9.9 us (8.7 with a slice's copies on one
+// scalar address); 128 x 128, 1101 x 3072 x 8192 33.7 -> 30.4 (one session each; 31.0 in another). What bounds the small tiles then is their copies, ~100 GB/s per CU (64 x 64: 0.16 us per 16 KiB slice);
+// more stages (6 to 8) measured slower, as did a k start that differs by block. The 256-row tiles
+// take the same cycles whatever the operands, the matrix cores busy 41% of them, but the clock follows the matrix cores' power:
+// 4096 x 3072 x 3072 28.8 us on zeros, 38.2 on random operands; 4096 x 8192 x 3072 65.1 and 92.7.
 template <int BM, int BN, int KB8, int NS, bool W4, int EPI, int MINB, int WGM, int NW, bool IL, int RA>
 __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ W, const float* __restrict__ as,
                                                       const float* __restrict__ ws, const half_t* __restrict__ gs, const half_t* __restrict__ bias,
@@ -470,12 +471,12 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm8_kernel(const int8_t* __re
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = wave / WGN, wn = wave % WGN;
 
     // Tile order: block ids go round-robin to the 8 XCDs, each with an L2 of its own. XCD x takes a contiguous eighth of the
-    // tiles in the order of strips STRIP tiles tall, column by column within a strip, so that the blocks it runs together
+    // tiles in the order of strips of at most 8 or 4 tiles' height (launch_gemm8), column by column within a strip, so that the blocks it runs together
     // cover a nearly square part of C and read few A and W panels through its L2. Any grid: ids that go round-robin over the
     // columns instead have every XCD read every panel (int8, us in plain order -> strips: 2821 x 11136 x 1792 in 128 x 128 tiles
     // 86.2 -> 62.8, 533 x 5952 x 12032 59.6 -> 43.5, in 64 x 128 96.2 -> 57.8, 641 x 704 x 10496 in 64 x 64 18.8 -> 16.6). Strips about 1024 rows tall measured best
     // of 1 to 16 tiles; the group-scaled 128-row tiles 4 tall (4096 x 12288 x 3072: 188.1 us against 190.3 at 8). The strips come from
-    // the launcher (tile_order): divided out here, they held back each workgroup's first copy by @@.
+    // the launcher (tile_order): divided out here, they held back each workgroup's first copy by 0.1-0.2 us (131 x 1024 x 192 5.75 us, 5.6 with factors).
     int bx, by;
     {
         const u32 n = gridDim.x * gridDim.y, id = blockIdx.y * gridDim.x + blockIdx.x, x = id % 8;
@@ -863,7 +864,9 @@ struct TileCost {
 
 // Least-squares fits to the measured times of 133 int8, 71 int4 and 74 group-scaled shapes (M 64-8192, N 512-12288, K
 // 1024-12288, and the DiT's own), every tile on every shape; the rule below then picks a tile within 0.8%, 2.0% and 1.1%
-// (geometric means) of the fastest one for the shape. No one tile does: 512 x 3072 x 3072 (int8) takes 9.9 us in
+// (geometric means) of the fastest one for the shape, and on 70, 40 and 50 random shapes that were not fitted within 0.5%, 3.2% and
+// 1.6% (at worst 3%, 21% and 8%: int4 542 x 2432 x 9728 27.9 us in 64 x 64, 23.0 in 64 x 128).
+// No one tile does, in one session: 512 x 3072 x 3072 (int8) 9.9 us in
 // 64 x 128 tiles, 13.0 in 128 x 128, 26 in 256 x 192 and 32 in 256 x 256 (24 to 32 workgroups for 256 CUs); 1101 x 3072 x 8192
 // 30.1 us in 128 x 128 and 59 in 256 x 192; 4096 x 3072 x 3072 38.5 us in 256 x 192 and 61 in 64 x 64.
 constexpr TileCost I8_TILES[] = {
