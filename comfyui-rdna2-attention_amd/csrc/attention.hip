@@ -806,9 +806,13 @@ static bool dma_ready(const void* p, long sb, long sh, long sl) { return ((uintp
 // still one per CU. B = 1, us unsplit / three groups of four, two and one waves: 24 x 1101 fp16 25.8 / 23.4, 31.1, 54.6, int8-QK
 // 24.9 / 23.9, 32.9, 52.0; 8 x 2000 (64-row grid: 256) 37.1 / 30.2, 26.5, 41.5; 2 x 9000 151 / 110, 181, 232; 4 x 1000 by 1152
 // keys 24.6 / 22.3, 17.6, 15.1. A split layout starts and ends ~1 us later than it would unsplit (more to copy first, O added up
-// at the end): 24 x 700 (22 tiles) breaks even, int8-QK at 27 (18.2 / 17.7 at 22, 23.9 / 24.9 at 35). Its sums are
-// those of another order, so the smallest calls, which must keep the bits that both unsplit layouts give (tests/test_gpu_attention.py),
-// stay with those: up to 736 keys, or 128-row workgroups for less than an eighth of the CUs.
+// at the end), which bounds the 128-row one: 24 x 700 (22 tiles) 16.7 / 15.6, int8-QK 17.9 / 17.8 there and 25.7 / 22.9 at 35 tiles.
+// Its sums are those of another order than the unsplit layouts', which agree bit for bit (tests/test_gpu_attention.py compares the
+// automatic choice with them). Up to 736 keys, or with 128-row workgroups for less than an eighth of the CUs, a call keeps the
+// unsplit bits, whatever its batch and heads; that line is drawn for the bits and costs time: 4 x 1000 by 576 13.8 us / 9.8 in 32-row
+// split workgroups, 8 x 500 12.9 / 9.6, 1 x 2000 36.5 / 21.4, 1 x 300 9.8 / 7.9. Past it a head's last bits depend on how many heads the
+// call has and, in two launches (below), on which it is: 24 x 1101 is split at batch 1 and not at batch 2. The results are equally far from
+// the 64-bit ones either way (24 x 1101 and 24 x 9293: relative error 2.9e-4 and 3.8e-4 before and after).
 // waves: 0 chooses so; 4 or 12 fixes an unsplit layout (12 needs Lq >= 384); -3, -6 or -12 (that many waves, in three key
 // groups) a split one (more than 64 keys, Q's rows 16-byte aligned).
 // Past one round of twelve-wave workgroups, a last round that is nearly empty costs as much as a full one (B = 1, 24 heads x 9293

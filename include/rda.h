@@ -115,10 +115,14 @@ int rda_attn_i8(const void* q, const void* workspace, const void* v, void* out, 
 /* rda_attn / rda_attn_i8 with the workgroup layout fixed: waves 4 (four-wave workgroups of 128 rows of one head) or 12
  * (twelve-wave workgroups of 384 rows of the (batch, head, row) range; needs Lq >= 384), which give the same bits; -12, -6 or
  * -3 (workgroups of 128, 64 or 32 rows of one head, that many waves in three groups that share the keys out; Lk > 64, q's
- * rows 16-byte aligned), which give the same bits as each other; or 0 for the choice rda_attn makes (split keys from 737
- * keys on where a grid of 128-row workgroups has at most one per CU and at least one for every eighth CU; else twelve waves
- * when Lq >= 384 and their grid covers at least two thirds of the CUs, the heads past its whole rounds in a second launch of
- * another layout where that is faster; else four). No reference counterpart: for tests and measurement of each layout. Other
+ * rows 16-byte aligned), which give the same bits as each other; or 0 for the choice rda_attn makes:
+ * - split keys from 737 keys on, where a grid of 128-row workgroups has at least one for every eighth CU and one of 32, 64 or
+ *   128 rows (the fewest that do) at most one per CU, q's rows being 16-byte aligned; int8-QK: 128 rows from 865 keys on;
+ * - else twelve waves when Lq >= 384 and their grid covers at least two thirds of the CUs, else four;
+ * - of more than one round of twelve-wave workgroups, the heads past the whole rounds in a second launch (split as above, there
+ *   without the eighth, or four waves), or, with few keys, all heads in four waves, where that is faster.
+ * The split sums are another order's: where that choice splits, a head's last bits depend on the call's batch and heads (for
+ * the same bits whatever they are, fix the layout). No reference counterpart: for tests and measurement of each layout. Other
  * values return 1. */
 int rda_attn_waves(const void* q, const void* k, const void* v, void* out, int B, int H, int Hkv, int Lq, int Lk, const long* strides, float scale,
                    int waves, void* stream);
