@@ -25,7 +25,7 @@ except ImportError:
     SingleStreamBlock = SwiGLU = None
 
 BLOCK_ROWS = 256  # rows of the GEMM's tallest tile (BM in csrc/gemm.hip); `quantize` pads its activations to it
-ROT_THREADS = 256  # threads per row of the rotate-quant pass (QT in csrc/quant.hip)
+ROT_THREADS = 256  # the reference's name; the library sizes its own launches (quant.hip: one to six waves per row)
 MIN_ROWS = 512  # Below this a GEMV-shaped call is better served by the original path.
 MAX_ROT_K = 16384  # Keeps the rotated row within the LDS of a workgroup.
 ROT_GROUP = 256

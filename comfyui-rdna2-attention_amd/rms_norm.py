@@ -14,7 +14,7 @@ except ImportError:
     comfy = None
     RMSNorm = None
 
-THREADS = 256  # NT in csrc/norm.hip
+THREADS = 256  # the reference's name; the library sizes its own launches (NT in csrc/norm.hip)
 HEAD_DIM = 128  # rows up to this width use 16 threads each (rms_norm_head)
 MAX_DIM = 8192  # 256 threads x 4 chunks x 8 values (rms_norm_row)
 
