@@ -72,8 +72,8 @@ __global__ __launch_bounds__(NT) void norm_kernel(const half_t* __restrict__ X, 
 
 // HPT heads of one token per 16 threads, H / HPT apart so that neighbouring slots still read neighbouring rows. What bounds
 // a row of one head is not its 512 bytes of x and y but the 1.5 KiB of weight and frequencies each head's threads load
-// again from L2; two heads share them. 4096 x 24 heads 13.2 -> 11.5 us (4.4 TB/s of x, y), 8192 x 24 22.3 -> 19.0; four
-// heads measured 11.3 and 19.5.
+// again from L2; two heads share them. Replayed on the same tensors: 4096 x 24 heads 12.5 -> 9.7 us, 8192 x 24 20.9 -> 18.1
+// (5.6 TB/s of x, y); in a block, after other work, 4096 x 24 takes 11.7. Four heads per 16 threads: 11.3 and 19.5 where two took 11.5 and 19.0.
 template <int HPT>
 __global__ __launch_bounds__(NT) void norm_rope_kernel(const half_t* __restrict__ X, const float* __restrict__ W, half_t* __restrict__ Y, int units, int L, int H,
                                                        long sb, long sh, long sl, float eps, const f4* __restrict__ F, long fb) {
