@@ -124,8 +124,8 @@ __device__ __forceinline__ int cvt_nearest_up(float x) {
 }
 
 // GROUP 256 or 128 rotates; GROUP 0 is quant_pack_a (no rotation, int8_gemm.hip:93-103). NW waves per row: the
-// launcher sizes it to the row (launch_rot_quant; K = 3072 keeps every lane of three waves busy in both passes: the kernel
-// is vector-ALU bound: 306 instructions per wave and 1024 values, 112 of them the butterflies, 411 before the conversions
+// launcher sizes it to the row (launch_rot_quant; K = 3072 keeps every lane of three waves busy in both passes: vector
+// instructions take 54% of its cycles, 77% with SwiGLU: 306 instructions per wave and 1024 values, 112 of them the butterflies, 411 before the conversions
 // were folded into multiply-adds: 4096 x 3072 10.8 -> 9.6 us (3.9 TB/s), SwiGLU 4096 x 8192 36.2 -> 34.0, MOD 4096 x 3072
 // 17.8 -> 15.8); MOD keeps 4 (QT threads), whose sum of squares follows the reference's thread order.
 // IL: the codes k-interleaved (each 8 values of k stored as their 4 even ones, then their 4 odd ones).
